@@ -188,7 +188,7 @@ struct RenderBuffers {
         }
         hits = HitDev{};
         dfree(shared.rad); dfree(shared.cnt); dfree(shared.direct); dfree(counts); dfree(list_off); dfree(list_scan_tmp); dfree(lists);
-        dfree(words); dfree(cam_states); dfree(cam_phi); dfree(rstat); dfree(tiles); dfree(chunkp); dfree(nch); dfree(chunk_off); dfree(tile_scan_tmp); dfree(partial); dfree(groups.keys); dfree(groups.vals); dfree(groups.tmp_k); dfree(groups.tmp_v); dfree(groups.hist); dfree(groups.nvalid); dfree(groups.chunkq); dfree(groups.stat); dfree(pass_dev); dfree(path_cell); dfree(path_ratio); dfree(pdep); dfree(doff); dfree(flags); dfree(ctr); dfree(raystripes); dfree(image);
+        dfree(words); dfree(cam_states); dfree(cam_phi); dfree(rstat); dfree(tiles); dfree(chunkp); dfree(nch); dfree(chunk_off); dfree(tile_scan_tmp); dfree(partial); dfree(groups.keys); dfree(groups.vals); dfree(groups.tmp_k); dfree(groups.tmp_v); dfree(groups.hist); dfree(groups.nvalid); dfree(groups.chunkq); dfree(groups.stat); dfree(groups.spheres); dfree(pass_dev); dfree(path_cell); dfree(path_ratio); dfree(pdep); dfree(doff); dfree(flags); dfree(ctr); dfree(raystripes); dfree(image);
         ready = false;
     }
 };
@@ -1032,6 +1032,7 @@ int sppm_begin(sppm_ctx* c) {
         (rc = dalloc(&R.groups.keys, np)) || (rc = dalloc(&R.groups.vals, np)) || (rc = dalloc(&R.groups.tmp_k, np)) ||
         (rc = dalloc(&R.groups.tmp_v, np)) || (rc = dalloc(&R.groups.hist, radix_hist_entries(np))) ||
         (rc = dalloc(&R.groups.nvalid, 1)) || (rc = dalloc(&R.groups.chunkq, STRIPE_INTS)) || (rc = dalloc(&R.groups.stat, 3 * (size_t)gather_group_count(np))) ||
+        (rc = dalloc(&R.groups.spheres, gather_sphere_entries(np))) ||
         (rc = dalloc(&R.pass_dev, 3)) ||
         (rc = dalloc(&R.image, np))) {
         R.release();
@@ -1922,6 +1923,7 @@ static int prepare_multi(sppm_batch* b) {
         J.order = gather_order(R.groups, R.np);
         J.nvalid = R.groups.nvalid;
         J.tiles = R.tiles;
+        J.spheres = R.groups.spheres;
         J.ntiles = gather_group_count(R.np);
         J.chunk_off = R.chunk_off;
         J.chunkp = R.chunkp;

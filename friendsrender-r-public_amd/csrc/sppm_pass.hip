@@ -15,7 +15,7 @@
 //   k_eye<W>         createHitpoints: one lane per pixel
 //   k_hit_keys ... k_gather_finish, k_group_stats
 //                    applyHitPointInfo + progressive update over Morton
-//                    groups of 64 hit points, chunked candidate lists
+//                    groups of 32 hit points, chunked candidate lists
 //   k_gather         the same with neighbour-list recording (tests)
 //   k_reconstruct    reconstructImageFromSharedPoints
 #include <hip/hip_runtime.h>
@@ -954,13 +954,13 @@ __global__ void __launch_bounds__(64) k_gather(HitDev H, SharedDev SH, GridDev G
 // ---------------------------------------------------------------------------
 // Load-balanced gather for the production pass (no neighbour lists).
 // Candidate counts per 8x8 tile vary by orders of magnitude (caustics), so:
-//   k_gather_plan    per tile: union cell box of its hit points and its
-//                    candidate count
+//   k_gather_plan    per tile: union cell box of its hit points, the
+//                    candidates of its rows (group_rows) and the query spheres
 //   k_chunk_size     candidates per chunk so that all chunks fit the buffer
 //   k_tile_chunks    chunks per tile
 //   scan             chunk offsets per tile
-//   k_gather_chunks  persistent waves take chunks of one tile's candidates,
-//                    stage them in LDS and write per-lane partial sums
+//   k_gather_chunks  persistent waves take chunks of one tile's candidates
+//                    and write per-lane partial sums
 //   k_gather_finish  per tile: partial sums in chunk order + the update
 // ---------------------------------------------------------------------------
 struct TileRange {
@@ -972,15 +972,13 @@ struct TileRange {
 // GATHER_GROUP per group.  World-space groups keep the union of their query
 // boxes close to one query box; screen tiles do not (a thin lens spreads a
 // tile's hit points over the circle of confusion).  The smaller the group,
-// the closer its union box to each member's own box: a wave holds each hit
-// point of a group in GATHER_PHASES lanes, and each of those lanes tests
-// every GATHER_PHASES-th staged photon.
-#ifndef SPPM_GATHER_GROUP
-#define SPPM_GATHER_GROUP 32
-#endif
-constexpr int GATHER_GROUP = SPPM_GATHER_GROUP;
+// the closer its union box to each member's own box.  A wave of the chunk
+// kernel tests 64 photons (one per lane) against one hit point of the group
+// after the other, then holds each hit point in GATHER_PHASES lanes, each of
+// which adds up the neighbours among its GATHER_GROUP of those photons.
+constexpr int GATHER_GROUP = 32;
 constexpr int GATHER_PHASES = 64 / GATHER_GROUP;
-static_assert(GATHER_GROUP == 16 || GATHER_GROUP == 32 || GATHER_GROUP == 64, "group of 16, 32 or 64 hit points");
+static_assert(GATHER_GROUP == 32, "one mask word per lane");
 __device__ __forceinline__ uint32_t spread10(uint32_t v) {
     v &= 0x3ffu;
     v = (v | (v << 16)) & 0x030000ffu;
@@ -1070,9 +1068,52 @@ __device__ __forceinline__ void load_gather_lane(const HitDev& H, const SharedDe
     }
 }
 
+// The photons of rows k0 .. k0 + 63 of a group's union box, one row per lane
+// (row k: y = T.y0 + k mod ny, z = T.z0 + k / ny): the cells between the
+// smallest and the largest x of those hit points whose own query box meets
+// the row; none if no box does.  A group that straddles a Morton boundary
+// has a union box far larger than the boxes in it (the whole scene, at
+// worst); its empty blocks of rows cost one ballot each, and no candidate.
+// r: the lane's own cell range (lanes past GATHER_GROUP are not read).
+// Called by the whole wave.
+struct RowSpan {
+    int start, len;
+};
+__device__ __forceinline__ RowSpan group_rows(const TileRange& T, int ny, int nrows, int k0, const int* r, bool active,
+                                              const GridParams& g, const int* __restrict__ cell_start) {
+    const int lane = threadIdx.x;
+    const int kl = min(k0 + 63, nrows - 1);
+    const int za = T.z0 + k0 / ny, zb = T.z0 + kl / ny;
+    const int ya = za == zb ? T.y0 + k0 % ny : T.y0, yb = za == zb ? T.y0 + kl % ny : T.y1;
+    unsigned long long pts = __ballot(active && lane < GATHER_GROUP && r[5] >= za && r[4] <= zb && r[3] >= ya && r[2] <= yb);
+    RowSpan s{0, 0};
+    if (pts == 0ull) return s;
+    const int k = k0 + lane;
+    const int y = T.y0 + k % ny, z = T.z0 + k / ny;
+    int x0 = 0x7fffffff, x1 = -1;
+    while (pts) {
+        const int i = __builtin_ctzll(pts);
+        pts &= pts - 1ull;
+        const int py = __builtin_amdgcn_readlane(r[2], i), ph = __builtin_amdgcn_readlane(r[3], i) - py;
+        const int pz = __builtin_amdgcn_readlane(r[4], i), pd = __builtin_amdgcn_readlane(r[5], i) - pz;
+        const bool in = ((unsigned)(y - py) <= (unsigned)ph) & ((unsigned)(z - pz) <= (unsigned)pd);
+        x0 = min(x0, in ? __builtin_amdgcn_readlane(r[0], i) : 0x7fffffff);
+        x1 = max(x1, in ? __builtin_amdgcn_readlane(r[1], i) : -1);
+    }
+    if (k < nrows && x1 >= x0) {
+        const int row = (z * g.ny + y) * g.nx;
+        s.start = cell_start[row + x0];
+        s.len = cell_start[row + x1 + 1] - s.start;
+    }
+    return s;
+}
+
+// Per group: its union cell box, its candidate count, and its hit points'
+// query spheres (centre, squared radius; -1: no hit point) for the chunk
+// kernel's scalar loads.
 __global__ void __launch_bounds__(64) k_gather_plan(HitDev H, SharedDev SH, GridDev G, const GridParams* __restrict__ gp,
                                                     const uint32_t* __restrict__ order, const int* __restrict__ nvalidp,
-                                                    TileRange* __restrict__ tiles) {
+                                                    TileRange* __restrict__ tiles, float4* __restrict__ spheres) {
     const int lane = threadIdx.x;
     const int p = lane < GATHER_GROUP ? group_pixel(order, *nvalidp, blockIdx.x * GATHER_GROUP + lane) : -1;
     const GridParams g = *gp;
@@ -1081,18 +1122,17 @@ __global__ void __launch_bounds__(64) k_gather_plan(HitDev H, SharedDev SH, Grid
     float4 sr;
     int r[6];
     load_gather_lane(H, SH, g, p, L, active, sr, r);
+    if (lane < GATHER_GROUP)
+        spheres[(size_t)blockIdx.x * GATHER_GROUP + lane] = make_float4(L.c.x, L.c.y, L.c.z, active ? L.R2 : -1.0f);
     TileRange T;
     T.x0 = -wave_max_i(active ? -r[0] : -0x7fffffff); T.x1 = wave_max_i(active ? r[1] : -1);
     T.y0 = -wave_max_i(active ? -r[2] : -0x7fffffff); T.y1 = wave_max_i(active ? r[3] : -1);
     T.z0 = -wave_max_i(active ? -r[4] : -0x7fffffff); T.z1 = wave_max_i(active ? r[5] : -1);
     int cand = 0;
     if (__ballot(active)) {
-        const int ny = T.y1 - T.y0 + 1, nrows = ny * (T.z1 - T.z0 + 1);
-        for (int k = lane; k < nrows; k += 64) {
-            const int y = T.y0 + k % ny, z = T.z0 + k / ny;
-            const int row = (z * g.ny + y) * g.nx;
-            cand += G.cell_start[row + T.x1 + 1] - G.cell_start[row + T.x0];
-        }
+        const int ny = __builtin_amdgcn_readfirstlane(T.y1 - T.y0 + 1);
+        const int nrows = __builtin_amdgcn_readfirstlane(ny * (T.z1 - T.z0 + 1));
+        for (int k0 = 0; k0 < nrows; k0 += 64) cand += group_rows(T, ny, nrows, k0, r, active, g, G.cell_start).len;
     } else {
         T.x0 = 0; T.x1 = -1; T.y0 = 0; T.y1 = -1; T.z0 = 0; T.z1 = -1;
     }
@@ -1102,7 +1142,13 @@ __global__ void __launch_bounds__(64) k_gather_plan(HitDev H, SharedDev SH, Grid
     if (lane == 0) tiles[blockIdx.x] = T;
 }
 
-// chunk size = max(1024, ceil(total / cap)) rounded to a multiple of 64
+// Candidates per chunk, a multiple of 64: about GATHER_CHUNKS_PER_WAVE chunks
+// for every persistent wave, between 128 (two batches of photons: below, a
+// chunk's own set-up would outweigh its work) and 1024 (above, a few heavy
+// groups would hold the last waves), or more if the chunks would not fit
+// their buffer (cap).  Always 1024 left a pass of few candidates on a few
+// hundred waves.
+constexpr int GATHER_CHUNKS_PER_WAVE = 2;
 __global__ void __launch_bounds__(256) k_chunk_size(const TileRange* __restrict__ tiles, int ntiles, int cap,
                                                     int* __restrict__ chunk, Counters* __restrict__ ctr) {
     __shared__ unsigned long long part[4];
@@ -1114,7 +1160,9 @@ __global__ void __launch_bounds__(256) k_chunk_size(const TileRange* __restrict_
     if (threadIdx.x == 0) {
         unsigned long long tot = part[0] + part[1] + part[2] + part[3];
         unsigned long long c = (tot + (unsigned long long)cap - 1) / (unsigned long long)cap;
-        if (c < 1024) c = 1024;
+        unsigned long long lo = tot / (unsigned long long)(GATHER_WAVES * GATHER_CHUNKS_PER_WAVE);
+        lo = lo < 128 ? 128 : lo > 1024 ? 1024 : lo;
+        if (c < lo) c = lo;
         c = (c + 63) & ~63ull;
         *chunk = (int)c;
         ctr->candidates += tot;
@@ -1130,40 +1178,64 @@ __global__ void k_tile_chunks(const TileRange* __restrict__ tiles, int ntiles, c
     nch[t] = (tiles[t].cand + c - 1) / c;
 }
 
-// The reference's two neighbour tests for one candidate, closed box
-// (kdtree.h:78-88) and the strict radius (SPPM.cpp:432), evaluated without
-// early exit.
-__device__ __forceinline__ bool in_query_nb(const GatherLane& L, const float4 pp) {
-    const bool box = (L.bbmin.x <= pp.x) & (pp.x <= L.bbmax.x) & (L.bbmin.y <= pp.y) & (pp.y <= L.bbmax.y) &
-                     (L.bbmin.z <= pp.z) & (pp.z <= L.bbmax.z);
-    const f3 d = mk(pp.x, pp.y, pp.z) - L.c;
-    return box & (norm2(d) < L.R2);
+// Transposes the 32 x 32 bit matrix that each half of the wave holds, a row
+// per lane: afterwards bit j of lane i is what bit i of lane j was.
+__device__ __forceinline__ uint32_t transpose32(uint32_t x, int lane) {
+#define SPPM_TRANSPOSE_STEP(S, M, OTHER)                                                       \
+    {                                                                                          \
+        const uint32_t v = (uint32_t)(OTHER);                                                  \
+        const bool up = (lane & S) != 0;                                                       \
+        const uint32_t keep = up ? ~M : M;                                                     \
+        const uint32_t rot = __builtin_amdgcn_alignbit(v, v, up ? S : 32 - S);                 \
+        x = (x & keep) | (rot & ~keep);                                                        \
+    }
+    SPPM_TRANSPOSE_STEP(16, 0x0000ffffu, __builtin_amdgcn_ds_swizzle((int)x, (16 << 10) | 0x1f))
+    SPPM_TRANSPOSE_STEP(8, 0x00ff00ffu, __builtin_amdgcn_ds_swizzle((int)x, (8 << 10) | 0x1f))
+    SPPM_TRANSPOSE_STEP(4, 0x0f0f0f0fu, __builtin_amdgcn_ds_swizzle((int)x, (4 << 10) | 0x1f))
+    SPPM_TRANSPOSE_STEP(2, 0x33333333u, __builtin_amdgcn_mov_dpp((int)x, 0x4e, 0xf, 0xf, true))  // quad_perm 2,3,0,1
+    SPPM_TRANSPOSE_STEP(1, 0x55555555u, __builtin_amdgcn_mov_dpp((int)x, 0xb1, 0xf, 0xf, true))  // quad_perm 1,0,3,2
+#undef SPPM_TRANSPOSE_STEP
+    return x;
 }
 
-// Persistent waves over the chunk list.  Per staged batch of 64 photons every
-// lane runs the two tests against its own hit point and lists the staged
-// photons that pass (LDS, one byte per entry, [entry][lane]); then every
-// lane walks its own list and accumulates W * BRDF * Flux / PDF
-// (SPPM.cpp:434-440).  Splitting the cheap tests from the BRDF evaluation
-// keeps the lanes of a wave busy in the second loop instead of evaluating
-// one lane's BRDF per candidate; each lane still adds its neighbours in
-// ascending candidate order.
+// Persistent waves over the chunk list.  A wave takes 64 candidate photons of
+// its chunk at a time, one per lane, filled across the rows of the group's
+// box, and tests them against the group's hit points one after the other:
+// the hit point's centre and squared radius are scalars (scalar loads), so a
+// test is nine vector instructions for 64 pairs and one or two to keep its
+// bit.  The bits are transposed from masks per photon to masks per hit point
+// (five exchange steps), and every lane walks the set bits of its mask and accumulates BRDF * Flux / PDF (SPPM.cpp:434-440), in ascending
+// candidate order; the photons' directions and fluxes are in LDS.
+//
+// The test is the strict radius alone (SPPM.cpp:432).  The reference also
+// tests a closed box first (kdtree.h:78-88), which the radius test implies in
+// float32 too: if p < fl(c - R) then p < c - R (p is a float and rounding is
+// monotonic), so fl(p - c)^2 >= fl(R * R) and the sum of squares is no less;
+// the upper sides alike, and with NaN both tests fail.
+//
+// Bound by vector instructions: about 10 per 64 pairs tested and 25 to 60 per
+// neighbour.  Before, a lane tested staged photons from LDS (22 instructions
+// and a 16-byte LDS read per pair, one row of cells at a time) over the whole
+// union box; a wave that entered a wide group walked its rows one dependent
+// load at a time.  The gather alone, mean of a render's first 8 passes: 64^2
+// pixels and 5k photons 0.504 -> 0.191 ms, 256^2 and 100k 0.688 -> 0.228,
+// 1024^2 and 1M (203k triangles) 2.715 -> 1.92, 1024^2 and 4M (caustics)
+// 12.76 -> 3.72.
 // The chunks of one scene's gather, claimed until its counters are exhausted.
 __device__ __forceinline__ void gather_chunks(HitDev H, SharedDev SH, GridDev G,
                                               const GridParams* __restrict__ gp, const uint32_t* __restrict__ order,
                                               const int* __restrict__ nvalidp, const TileRange* __restrict__ tiles,
-                                              int ntiles, const int* __restrict__ chunk_off,
-                                              const int* __restrict__ chunkp, int* __restrict__ queue,
-                                              float4* __restrict__ partial, unsigned long long* __restrict__ pdep,
-                                              PairRecord rec) {
+                                              const float4* __restrict__ spheres, int ntiles,
+                                              const int* __restrict__ chunk_off, const int* __restrict__ chunkp,
+                                              int* __restrict__ queue, float4* __restrict__ partial,
+                                              unsigned long long* __restrict__ pdep, PairRecord rec) {
     // LDS of the loop (one wave per block; each kernel that inlines this
     // function gets its own arrays)
-    __shared__ float4 s_pos[64], s_flux[64], s_dir[64];
-    __shared__ unsigned char s_hit[64 * 64];
-    __shared__ int s_cnt[64];  // hit points of this group gathering each staged photon (guided emission)
+    __shared__ float4 s_flux[64], s_dir[64];
+    __shared__ int s_id[64];  // flattened photon indices (pair recording)
     const int lane = threadIdx.x;
     const int hl = lane % GATHER_GROUP;   // the lane's hit point in the group
-    const int ph = lane / GATHER_GROUP;   // the lane tests staged photons ph, ph + GATHER_PHASES, ...
+    const int ph = lane / GATHER_GROUP;   // the lane adds up staged photons ph * GATHER_GROUP ...
     const int total = chunk_off[ntiles];
     const int CH = *chunkp;
     const int nvalid = *nvalidp;
@@ -1176,92 +1248,109 @@ __device__ __forceinline__ void gather_chunks(HitDev H, SharedDev SH, GridDev G,
     for (;;) {
         int ch = 0;
         if (!stripe_claim_rr(queue, total, cur, &ch)) break;
+        ch = __builtin_amdgcn_readfirstlane(ch);
         // owning tile: last t with chunk_off[t] <= ch
         int lo = 0, hi = ntiles;
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
             if (chunk_off[mid] <= ch) lo = mid; else hi = mid;
         }
-        const int t = lo;
+        const int t = __builtin_amdgcn_readfirstlane(lo);
         const TileRange T = tiles[t];
+        // constant address space: scalar loads also where the pointer comes from a job table
+        typedef float sphere_t __attribute__((ext_vector_type(4)));
+        typedef const sphere_t __attribute__((address_space(4))) * sphere_ptr;
+        const sphere_ptr sph = (sphere_ptr)(uintptr_t)(spheres + (size_t)t * GATHER_GROUP);
         const int p = group_pixel(order, nvalid, t * GATHER_GROUP + hl);
         GatherLane L;
         bool active;
         float4 sr;
         int r[6];
         load_gather_lane(H, SH, g, p, L, active, sr, r);
-        const long long first = (long long)(ch - chunk_off[t]) * CH;
-        const long long last = first + CH < T.cand ? first + CH : T.cand;
+        const float on = dot(L.outd, L.N);
+        // the pixel weight multiplies the sum, unless it is not finite (then
+        // every term, as W * BRDF * Flux / PDF gives NaN for a zero factor)
+        const bool wfin = isfinite(L.wgt.x) && isfinite(L.wgt.y) && isfinite(L.wgt.z);
+        const int first = (ch - chunk_off[t]) * CH;
+        const int last = T.cand - first > CH ? first + CH : T.cand;
         const int ny = T.y1 - T.y0 + 1, nrows = ny * (T.z1 - T.z0 + 1);
-        long long acc = 0;  // candidates before the current row
-        for (int k = 0; k < nrows && acc < last; ++k) {
-            const int y = T.y0 + k % ny, z = T.z0 + k / ny;
-            const int row = (z * g.ny + y) * g.nx;
-            const int qa = G.cell_start[row + T.x0];
-            const int qb = G.cell_start[row + T.x1 + 1];
-            const long long len = qb - qa;
-            const long long s0 = first > acc ? first - acc : 0;
-            const long long s1 = last - acc < len ? last - acc : len;
-            acc += len;
-            if (s0 >= s1) continue;
-            const bool mine = active && z >= r[4] && z <= r[5] && y >= r[2] && y <= r[3];
-            for (long long base = qa + s0; base < qa + s1; base += 64) {
-                const long long q = base + lane;
-                if (q < qa + s1) {
-                    s_pos[lane] = G.pos[q];
-                    s_flux[lane] = G.flux[q];
-                    s_dir[lane] = G.dir[q];
+        int acc = 0;  // candidates before the current block of rows
+        for (int k0 = 0; k0 < nrows && acc < last; k0 += 64) {
+            const RowSpan row = group_rows(T, ny, nrows, k0, r, active, g, G.cell_start);
+            int incl = row.len;
+            for (int off = 1; off < 64; off <<= 1) {
+                const int v = __shfl_up(incl, off, 64);
+                if (lane >= off) incl += v;
+            }
+            const int tot = __builtin_amdgcn_readlane(incl, 63);
+            const int b0 = first > acc ? first - acc : 0;
+            const int b1 = last - acc < tot ? last - acc : tot;
+            acc += tot;
+            const int roff = row.start - (incl - row.len);  // candidate c of the row is photon roff + c
+            for (int base = b0; base < b1; base += 64) {
+                const int n = min(64, b1 - base);
+                const int c = base + min(lane, n - 1);
+                // the first row that ends past c; mostly one row holds all 64
+                const int r0 = __builtin_ctzll(__ballot(incl > base));
+                int q;
+                if (__builtin_amdgcn_readlane(incl, r0) >= base + n) {
+                    q = __builtin_amdgcn_readlane(roff, r0) + c;
+                } else {
+                    int k = 0;
+#pragma unroll
+                    for (int s = 32; s > 0; s >>= 1)
+                        if (__shfl(incl, k + s - 1, 64) <= c) k += s;
+                    q = __shfl(roff, k, 64) + c;
                 }
-                if (pdep) s_cnt[lane] = 0;
+                const float4 pp = G.pos[q], pf = G.flux[q], pd = G.dir[q];
+                const float inv = __builtin_amdgcn_rcpf(pf.w);
+                s_flux[lane] = make_float4(pf.x * inv, pf.y * inv, pf.z * inv, 0.0f);
+                s_dir[lane] = make_float4(pd.x, pd.y, pd.z, pp.w);
+                if (rec.pairs) s_id[lane] = __float_as_int(pd.w);
                 __syncthreads();
-                const int n = (int)((qa + s1 - base) < 64 ? (qa + s1 - base) : 64);
-                int nh = 0;
-                if (mine) {
-                    // four of this lane's staged photons per step, no branches: the list
-                    // slot nh is written every time and kept only when the photon passes
-                    // (nh <= the photons tested so far, so the slot stays below 64)
-                    int j = ph;
-                    for (; j + 3 * GATHER_PHASES < n; j += 4 * GATHER_PHASES) {
-                        const float4 p0 = s_pos[j], p1 = s_pos[j + GATHER_PHASES];
-                        const float4 p2 = s_pos[j + 2 * GATHER_PHASES], p3 = s_pos[j + 3 * GATHER_PHASES];
-                        const bool h0 = in_query_nb(L, p0), h1 = in_query_nb(L, p1);
-                        const bool h2 = in_query_nb(L, p2), h3 = in_query_nb(L, p3);
-                        s_hit[nh * 64 + lane] = (unsigned char)j;
-                        nh += h0;
-                        s_hit[nh * 64 + lane] = (unsigned char)(j + GATHER_PHASES);
-                        nh += h1;
-                        s_hit[nh * 64 + lane] = (unsigned char)(j + 2 * GATHER_PHASES);
-                        nh += h2;
-                        s_hit[nh * 64 + lane] = (unsigned char)(j + 3 * GATHER_PHASES);
-                        nh += h3;
-                    }
-                    for (; j < n; j += GATHER_PHASES) {
-                        s_hit[nh * 64 + lane] = (unsigned char)j;
-                        nh += in_query_nb(L, s_pos[j]);
-                    }
+                uint32_t mask = 0;  // bit i: hit point i gathers this lane's photon
+                // lanes past n hold no candidate
+                const f3 pos = mk(lane < n ? pp.x : __builtin_inff(), pp.y, pp.z);
+#pragma unroll 16
+                for (int i = GATHER_GROUP - 1; i >= 0; --i) {
+                    const sphere_t sp = sph[i];
+                    mask = (mask << 1) + (norm2(pos - mk(sp.x, sp.y, sp.z)) < sp.w ? 1u : 0u);
                 }
+                const int cnt = __popc(mask);  // hit points of the group that gather this lane's photon
+                mask = transpose32(mask, lane);  // bit j: staged photon ph * 32 + j is gathered by this lane's hit point
+                const int nh = __popc(mask);
                 L.M += nh;
                 if (rec.pairs) {
                     // recording (parity tests): this lane's neighbours among the staged
                     // photons, appended at a wave-wide prefix of the lanes' counts
-                    int incl = nh;
+                    int incl_h = nh;
                     for (int off = 1; off < 64; off <<= 1) {
-                        const int v = __shfl_up(incl, off, 64);
-                        if (lane >= off) incl += v;
+                        const int v = __shfl_up(incl_h, off, 64);
+                        if (lane >= off) incl_h += v;
                     }
-                    const int tot = __shfl(incl, 63, 64);
-                    unsigned long long base = 0;
-                    if (lane == 0 && tot > 0) base = atomicAdd(rec.count, (unsigned long long)tot);
-                    base = __shfl(base, 0, 64) + (unsigned long long)(incl - nh);
-                    for (int e = 0; e < nh; ++e)
-                        if ((long long)(base + e) < rec.cap)
-                            rec.pairs[base + e] = make_int2(p, __float_as_int(s_dir[s_hit[e * 64 + lane]].w));
+                    const int toth = __shfl(incl_h, 63, 64);
+                    unsigned long long at = 0;
+                    if (lane == 0 && toth > 0) at = atomicAdd(rec.count, (unsigned long long)toth);
+                    at = __shfl(at, 0, 64) + (unsigned long long)(incl_h - nh);
+                    uint32_t mm = mask;
+                    for (int e = 0; e < nh; ++e) {
+                        const int j = ph * GATHER_GROUP + __builtin_ctz(mm);
+                        mm &= mm - 1u;
+                        if ((long long)(at + e) < rec.cap) rec.pairs[at + e] = make_int2(p, s_id[j]);
+                    }
                 }
-                const float on = dot(L.outd, L.N);
-                for (int e = 0; e < nh; ++e) {
-                    const int j = s_hit[e * 64 + lane];
-                    const float4 pp = s_pos[j], pf = s_flux[j], pd = s_dir[j];
-                    const f3 indir = mk(pd.x, pd.y, pd.z);
+                if (pdep) {
+                    // training signal of the emission proposal: hit points reached x photon power
+                    if (cnt > 0) {
+                        const float d = (float)cnt * (0.2126f * pf.x + 0.7152f * pf.y + 0.0722f * pf.z) / pf.w;
+                        if (d > 0.0f && d < 3.0e38f) atomicAdd(&pdep[__float_as_int(pd.w)], guide_fix(d));
+                    }
+                }
+                while (mask) {
+                    const int j = ph * GATHER_GROUP + __builtin_ctz(mask);
+                    mask &= mask - 1u;
+                    const float4 fl = s_flux[j], dr = s_dir[j];
+                    const f3 indir = mk(dr.x, dr.y, dr.z);
                     const float din = dot(indir, L.N);
                     float b;
                     if (L.kind == SPPM_MAT_DIFFUSE) {
@@ -1271,27 +1360,19 @@ __device__ __forceinline__ void gather_chunks(HitDev H, SharedDev SH, GridDev G,
                         const float co = din < 0 ? on : -on;
                         b = (fabs_(din) > LO_1EM4 && co > LO_1EM4) ? 1.0f / SPPM_PI : 0.0f;
                     } else {
-                        const float Io = near1(pp.w) ? L.ior : 1.0f;
+                        const float Io = near1(dr.w) ? L.ior : 1.0f;
                         const f3 nrm = din < 0 ? L.N : -L.N;
-                        FParam fp{indir, L.outd, nrm, pp.w, Io, L.rough, L.absorb, L.refl};
+                        FParam fp{indir, L.outd, nrm, dr.w, Io, L.rough, L.absorb, L.refl};
                         b = gather_brdf(L.kind, fp);
                     }
-                    L.add = L.add + ((L.wgt * b) * mk(pf.x, pf.y, pf.z)) * __builtin_amdgcn_rcpf(pf.w);
-                    // guided emission: per staged photon, the hit points that gather it
-                    if (pdep) atomicAdd(&s_cnt[j], 1);
-                }
-                if (pdep) {
-                    // training signal of the emission proposal: hit points reached x photon power
-                    __syncthreads();
-                    if (lane < n && s_cnt[lane] > 0) {
-                        const float4 pf = s_flux[lane];
-                        const float d = (float)s_cnt[lane] * (0.2126f * pf.x + 0.7152f * pf.y + 0.0722f * pf.z) / pf.w;
-                        if (d > 0.0f && d < 3.0e38f) atomicAdd(&pdep[__float_as_int(s_dir[lane].w)], guide_fix(d));
-                    }
+                    f3 term = mk(fl.x, fl.y, fl.z) * b;
+                    if (!wfin) term = L.wgt * term;
+                    L.add = L.add + term;
                 }
                 __syncthreads();
             }
         }
+        if (wfin) L.add = L.wgt * L.add;
         // the hit point's sums over its lanes, in phase order (deterministic)
         f3 tot = mk(0.0f, 0.0f, 0.0f);
         int Mt = 0;
@@ -1313,11 +1394,12 @@ constexpr int GATHER_WAVES_PER_SIMD = 4;
 __global__ void __launch_bounds__(64) k_gather_chunks(HitDev H, SharedDev SH, GridDev G,
                                                       const GridParams* __restrict__ gp,
                                                       const uint32_t* __restrict__ order, const int* __restrict__ nvalidp,
-                                                      const TileRange* __restrict__ tiles, int ntiles,
+                                                      const TileRange* __restrict__ tiles,
+                                                      const float4* __restrict__ spheres, int ntiles,
                                                       const int* __restrict__ chunk_off, const int* __restrict__ chunkp,
                                                       int* __restrict__ queue, float4* __restrict__ partial,
                                                       unsigned long long* __restrict__ pdep, PairRecord rec) {
-    gather_chunks(H, SH, G, gp, order, nvalidp, tiles, ntiles, chunk_off, chunkp, queue, partial, pdep, rec);
+    gather_chunks(H, SH, G, gp, order, nvalidp, tiles, spheres, ntiles, chunk_off, chunkp, queue, partial, pdep, rec);
 }
 
 // The gather chunks of every scene of a batch (see k_photon_multi).
@@ -1328,7 +1410,7 @@ __global__ void __launch_bounds__(64, GATHER_WAVES_PER_SIMD) k_gather_chunks_mul
         const int s = __builtin_amdgcn_readfirstlane(home + k < njobs ? home + k : home + k - njobs);
         const GatherJob& J = jobs[s];
         if (scene_done(J.queue)) continue;
-        gather_chunks(J.H, J.SH, J.G, J.gp, J.order, J.nvalid, J.tiles, J.ntiles, J.chunk_off, J.chunkp, J.queue,
+        gather_chunks(J.H, J.SH, J.G, J.gp, J.order, J.nvalid, J.tiles, J.spheres, J.ntiles, J.chunk_off, J.chunkp, J.queue,
                       J.partial, J.pdep, J.rec);
         scene_mark_done(J.queue);
     }
@@ -1674,7 +1756,7 @@ const uint32_t* launch_gather_plan(const HitDev& H, const SharedDev& SH, const G
     const SortResult sr = radix_sort_pairs(gb.keys, gb.vals, gb.tmp_k, gb.tmp_v, gb.hist, np, 31, st);
     hipLaunchKernelGGL(k_count_valid, dim3(1), dim3(64), 0, st, sr.keys, np, gb.nvalid);
     const uint32_t* order = sr.vals;  // == gather_order(gb, np)
-    hipLaunchKernelGGL(k_gather_plan, dim3(ntiles), dim3(64), 0, st, H, SH, G, gp, order, gb.nvalid, tiles);
+    hipLaunchKernelGGL(k_gather_plan, dim3(ntiles), dim3(64), 0, st, H, SH, G, gp, order, gb.nvalid, tiles, gb.spheres);
     hipLaunchKernelGGL(k_chunk_size, dim3(1), dim3(256), 0, st, tiles, ntiles, cap, chunkp, ctr);
     hipLaunchKernelGGL(k_tile_chunks, dim3((ntiles + 1 + 255) / 256), dim3(256), 0, st, tiles, ntiles, chunkp, nch);
     exclusive_scan(nch, chunk_off, ntiles + 1, nullptr, scan_tmp, st);
@@ -1686,7 +1768,7 @@ void launch_gather_run(const HitDev& H, const SharedDev& SH, const GridDev& G, c
                        const int* chunk_off, float4* partial, unsigned long long* pdep, const PairRecord& rec,
                        hipStream_t st) {
     hipLaunchKernelGGL(k_gather_chunks, dim3(GATHER_WAVES), dim3(64), 0, st, H, SH, G, gp, order, gb.nvalid, tiles,
-                       gather_group_count(np), chunk_off, chunkp, gb.chunkq, partial, pdep, rec);
+                       gb.spheres, gather_group_count(np), chunk_off, chunkp, gb.chunkq, partial, pdep, rec);
 }
 void launch_gather_finish(const HitDev& H, const SharedDev& SH, int np, const uint32_t* order, const GroupBuffers& gb,
                           float alpha, const int* chunk_off, const float4* partial, int* counts,
@@ -1747,6 +1829,7 @@ const uint32_t* gather_order(const GroupBuffers& gb, int np) {
 }
 int gather_tile_count(int W, int Hh) { return ((W + 7) >> 3) * ((Hh + 7) >> 3); }
 int gather_group_count(int np) { return (np + GATHER_GROUP - 1) / GATHER_GROUP; }
+size_t gather_sphere_entries(int np) { return (size_t)gather_group_count(np) * GATHER_GROUP; }
 size_t gather_tile_bytes() { return sizeof(TileRange); }
 
 void launch_reconstruct(const SharedDev& SH, int np, long long total, int passes, float4* out, hipStream_t st) {
