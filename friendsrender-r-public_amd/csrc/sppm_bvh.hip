@@ -14,6 +14,7 @@
 // Closest-hit results do not depend on the tree (ties go to the lowest facet
 // id), so the build is free to optimise traversal cost.
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <string.h>
@@ -154,10 +155,13 @@ __global__ void k_refit(const float4* __restrict__ tbmin, const float4* __restri
 }
 
 
-__global__ void k_tri_reorder(const float* __restrict__ pos, const uint32_t* __restrict__ order, int n,
-                              float4* __restrict__ tri) {
+__global__ void k_tri_reorder(const float* __restrict__ pos, const uint32_t* __restrict__ order,
+                              int n, float4* __restrict__ tri) {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
+    if (k >= n) {
+        if (k < n + TRI_PAD) tri[3 * k] = tri[3 * k + 1] = tri[3 * k + 2] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        return;
+    }
     uint32_t f = order[k];
     const float* p = pos + 9 * (size_t)f;
     float v0x = p[0], v0y = p[1], v0z = p[2];
@@ -407,11 +411,71 @@ namespace {
 constexpr float DP_C_NODE = 1.0f;
 constexpr float DP_C_TRI = 0.15f;
 constexpr float DP_C_LEAF = 0.5f;  // entering a leaf (pop, loop set-up): 4.03 ms per pass, 4.07 without
-constexpr int DP_LEAF_MAX = 8;  // a leaf reference holds count - 1 in 3 bits
+constexpr int DP_LEAF_MAX = 8;  // a leaf reference holds count - 1 in 3 bits, eight leaves' ends fit 7
+
+struct WideChild {
+    float4 lo, hi;
+    int count;  // triangles of a leaf; 0: inner
+};
+// A float whose bits above 21 are kept, not below v.
+float frame_step(double v) {
+    float f = (float)v;
+    if ((double)f < v) f = nextafterf(f, 3.0e38f);
+    uint32_t b;
+    memcpy(&b, &f, 4);
+    b = (b + 0x1fffffu) & ~0x1fffffu;
+    if (b < 0x00800000u) b = 0x00800000u;
+    memcpy(&f, &b, 4);
+    return f;
+}
+// One node (layout: sppm_layout.h) of n children, leaves first.  The boxes are widened by a
+// few roundings of the device's plane distances, then rounded outwards.
+void encode_node(uint32_t* w, int W, const WideChild* c, int n, uint32_t child_base, uint32_t tri_base) {
+    unsigned char* const meta = reinterpret_cast<unsigned char*>(w + 6);
+    unsigned char* const planes = reinterpret_cast<unsigned char*>(w + NODE_PLANES(W));
+    memset(w, 0, sizeof(uint32_t) * node_words(W));
+    w[4] = child_base;
+    w[5] = tri_base;
+    int inner = 0, end = 0;
+    for (int k = 0; k < n; ++k) meta[k] = (unsigned char)(c[k].count ? NODE_LEAF | (uint32_t)(end += c[k].count) : (uint32_t)inner++);
+    for (int k = n; k < W; ++k) meta[k] = (unsigned char)(inner ? (uint32_t)(inner - 1) : NODE_LEAF | (uint32_t)++end);
+    for (int a = 0; a < 3; ++a) {
+        // vertices that are not finite meet no ray; they only must not spoil the frame
+        auto fin = [](float v) { return fmin(fmax((double)v, -1e30), 1e30); };
+        auto lo = [&](int k) { return fin(a == 0 ? c[k].lo.x : (a == 1 ? c[k].lo.y : c[k].lo.z)); };
+        auto hi = [&](int k) { return fin(a == 0 ? c[k].hi.x : (a == 1 ? c[k].hi.y : c[k].hi.z)); };
+        double mn = lo(0), mx = hi(0);
+        for (int k = 1; k < n; ++k) {
+            mn = lo(k) < mn ? lo(k) : mn;
+            mx = hi(k) > mx ? hi(k) : mx;
+        }
+        const double eps = (fmax(fabs(mn), fabs(mx)) + (mx - mn)) * 0x1p-23;
+        float org = (float)(mn - eps);
+        if ((double)org > mn - eps) org = nextafterf(org, -3.0e38f);
+        const float step = frame_step((mx + eps - (double)org) / 255.0);
+        memcpy(w + a, &org, 4);
+        uint32_t b;
+        memcpy(&b, &step, 4);
+        w[3] |= (b >> 21) << (10 * a);
+        for (int k = 0; k < W; ++k) {
+            double ql = 255.0, qh = 0.0;
+            if (k < n) {
+                ql = floor((lo(k) - eps - (double)org) / (double)step);
+                qh = ceil((hi(k) + eps - (double)org) / (double)step);
+                ql = ql < 0.0 ? 0.0 : (ql > 255.0 ? 255.0 : ql);
+                qh = qh < 0.0 ? 0.0 : (qh > 255.0 ? 255.0 : qh);
+            }
+            planes[(2 * a) * W + k] = (unsigned char)ql;
+            planes[(2 * a + 1) * W + k] = (unsigned char)qh;
+        }
+    }
+}
+// nodes: the encoded wide nodes.  perm: leaf triangle i is triangle perm[i] of
+// the binary tree's order.
 int collapse_dp(const std::vector<int2>& child, const std::vector<int2>& range, const std::vector<float4>& bmin,
-                const std::vector<float4>& bmax, int n, int root, int W, std::vector<float>& nodes) {
+                const std::vector<float4>& bmax, int n, int root, int W, std::vector<uint32_t>& nodes, std::vector<uint32_t>& perm) {
     const int NN = 2 * n - 1;
-    const int NF = node_floats(W);
+    const int NF = node_words(W);
     auto area = [&](int m) {
         const float x = bmax[m].x - bmin[m].x, y = bmax[m].y - bmin[m].y, z = bmax[m].z - bmin[m].z;
         return x * y + y * z + z * x;
@@ -496,42 +560,37 @@ int collapse_dp(const std::vector<int2>& child, const std::vector<int2>& range, 
         }
     };
     nodes.clear();
+    perm.clear();
     std::vector<int> queue{root};
     size_t head = 0;
     while (head < queue.size()) {
         const int m = queue[head];
         const int w = (int)head;
         ++head;
-        nodes.resize((size_t)(w + 1) * NF, 0.0f);
-        float* nd = nodes.data() + (size_t)w * NF;
-        uint32_t cref[8];
         ent.clear();
         // a wide node splits its W slots between its two binary children
         const int k = dk[(size_t)m * 9 + W];
         collect(child[m].x, k);
         collect(child[m].y, W - k);
         if ((int)ent.size() > W) return -1;
-        for (int c = 0; c < W; ++c) {
-            if (c < (int)ent.size()) {
-                const int x = ent[c];
-                nd[0 * W + c] = bmin[x].x; nd[1 * W + c] = bmin[x].y; nd[2 * W + c] = bmin[x].z;
-                nd[3 * W + c] = bmax[x].x; nd[4 * W + c] = bmax[x].y; nd[5 * W + c] = bmax[x].z;
-                const int p = tris(x);
-                if (x >= n - 1 || how[(size_t)x * 9 + 1] == 0) {
-                    if (p > DP_LEAF_MAX) return -1;
-                    const int first = x >= n - 1 ? x - (n - 1) : range[x].x;
-                    cref[c] = LEAF_BIT | ((uint32_t)first << 3) | (uint32_t)(p - 1);
-                } else {
-                    cref[c] = (uint32_t)queue.size();
-                    queue.push_back(x);
-                }
-            } else {
-                nd[0 * W + c] = 1e30f; nd[1 * W + c] = 1e30f; nd[2 * W + c] = 1e30f;
-                nd[3 * W + c] = -1e30f; nd[4 * W + c] = -1e30f; nd[5 * W + c] = -1e30f;
-                cref[c] = EMPTY_CHILD;
-            }
+        const uint32_t child_base = (uint32_t)queue.size(), tri_base = (uint32_t)perm.size();
+        WideChild wc[8];
+        int nc = 0;
+        for (int x : ent) {
+            if (x < n - 1 && how[(size_t)x * 9 + 1] != 0) continue;
+            const int p = tris(x);
+            if (p > DP_LEAF_MAX) return -1;
+            const int f = x >= n - 1 ? x - (n - 1) : range[x].x;
+            wc[nc++] = WideChild{bmin[x], bmax[x], p};
+            for (int t = 0; t < p; ++t) perm.push_back((uint32_t)(f + t));
         }
-        memcpy(nd + 6 * W, cref, sizeof(uint32_t) * W);
+        for (int x : ent) {
+            if (x >= n - 1 || how[(size_t)x * 9 + 1] == 0) continue;
+            wc[nc++] = WideChild{bmin[x], bmax[x], 0};
+            queue.push_back(x);
+        }
+        nodes.resize((size_t)(w + 1) * NF);
+        encode_node(nodes.data() + (size_t)w * NF, W, wc, nc, child_base, tri_base);
     }
     return (int)queue.size();
 }
@@ -541,13 +600,14 @@ int build_bvh(const float* pos, int n, int width, bool sah, hipStream_t st, BvhR
               size_t errlen) {
     const int TB = 256;
     const int G = (n + TB - 1) / TB;
-    const int NF = node_floats(width);
+    const int NF = node_words(width);
     float4 *tbmin = nullptr, *tbmax = nullptr, *nbmin = nullptr, *nbmax = nullptr;
     uint32_t *cb = nullptr, *keys = nullptr, *vals = nullptr, *tk = nullptr, *tv = nullptr, *hist = nullptr;
     int2 *child = nullptr, *range = nullptr;
     int *parent = nullptr, *flag = nullptr, *counters = nullptr;
     SahSeg *sa = nullptr, *sb = nullptr;
     int root_id = 0;
+    std::vector<uint32_t> hn;  // the wide nodes
     int nint = n > 1 ? n - 1 : 1;
     int maxw = n > 1 ? n - 1 : 1;
     int hcnt[2];
@@ -581,8 +641,8 @@ int build_bvh(const float* pos, int n, int width, bool sah, hipStream_t st, BvhR
         HIPCHK(hipMalloc(&sa, sizeof(SahSeg) * (size_t)n));
         HIPCHK(hipMalloc(&sb, sizeof(SahSeg) * (size_t)n));
     }
-    HIPCHK(hipMalloc(&out->nodes, sizeof(float) * NF * (size_t)maxw));
-    HIPCHK(hipMalloc(&out->tri, sizeof(float4) * 3 * (size_t)n));
+    HIPCHK(hipMalloc(&out->nodes, sizeof(uint32_t) * NF * (size_t)maxw));
+    HIPCHK(hipMalloc(&out->tri, sizeof(float4) * 3 * ((size_t)n + TRI_PAD)));
     {
         uint32_t init[6] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0u, 0u, 0u};
         HIPCHK(hipMemcpyAsync(cb, init, sizeof(init), hipMemcpyHostToDevice, st));
@@ -652,24 +712,16 @@ int build_bvh(const float* pos, int n, int width, bool sah, hipStream_t st, BvhR
     }
     hipLaunchKernelGGL(k_refit, dim3(G), dim3(TB), 0, st, tbmin, tbmax, vals, n, child, parent, nbmin, nbmax, flag,
                        root_id);
-    hipLaunchKernelGGL(k_tri_reorder, dim3(G), dim3(TB), 0, st, pos, vals, n, out->tri);
     HIPCHK(hipGetLastError());
     if (n == 1) {
         // one leaf under a single wide node
-        std::vector<float> nd(NF, 0.0f);
-        float4 lo, hi;
-        HIPCHK(hipMemcpyAsync(&lo, nbmin, sizeof(float4), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(&hi, nbmax, sizeof(float4), hipMemcpyDeviceToHost, st));
+        WideChild c{};
+        HIPCHK(hipMemcpyAsync(&c.lo, nbmin, sizeof(float4), hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(&c.hi, nbmax, sizeof(float4), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
-        for (int k = 0; k < width; ++k) {
-            bool real = k == 0;
-            nd[0 * width + k] = real ? lo.x : 1e30f; nd[1 * width + k] = real ? lo.y : 1e30f;
-            nd[2 * width + k] = real ? lo.z : 1e30f; nd[3 * width + k] = real ? hi.x : -1e30f;
-            nd[4 * width + k] = real ? hi.y : -1e30f; nd[5 * width + k] = real ? hi.z : -1e30f;
-            uint32_t r = real ? (LEAF_BIT | 0u) : EMPTY_CHILD;
-            memcpy(&nd[6 * width + k], &r, 4);
-        }
-        HIPCHK(hipMemcpyAsync(out->nodes, nd.data(), sizeof(float) * NF, hipMemcpyHostToDevice, st));
+        c.count = 1;
+        hn.resize(NF);
+        encode_node(hn.data(), width, &c, 1, 0u, 0u);
         out->nnodes = 1;
         depth = 1;
     } else {
@@ -680,23 +732,28 @@ int build_bvh(const float* pos, int n, int width, bool sah, hipStream_t st, BvhR
         HIPCHK(hipMemcpy(hr.data(), range, sizeof(int2) * hr.size(), hipMemcpyDeviceToHost));
         HIPCHK(hipMemcpy(hlo.data(), nbmin, sizeof(float4) * hlo.size(), hipMemcpyDeviceToHost));
         HIPCHK(hipMemcpy(hhi.data(), nbmax, sizeof(float4) * hhi.size(), hipMemcpyDeviceToHost));
-        std::vector<float> hn;
-        const int nw = collapse_dp(hc, hr, hlo, hhi, n, root_id, width, hn);
-        if (nw <= 0 || nw > maxw) {
+        std::vector<uint32_t> perm;
+        const int nw = collapse_dp(hc, hr, hlo, hhi, n, root_id, width, hn, perm);
+        if (nw <= 0 || nw > maxw || (int)perm.size() != n) {
             snprintf(err, errlen, "BVH collapse failed (%d nodes)", nw);
             goto fail;
         }
-        HIPCHK(hipMemcpy(out->nodes, hn.data(), sizeof(float) * hn.size(), hipMemcpyHostToDevice));
+        // the facets in the leaves' order
+        std::vector<uint32_t> hv(n), ho(n);
+        HIPCHK(hipMemcpy(hv.data(), vals, sizeof(uint32_t) * n, hipMemcpyDeviceToHost));
+        for (int t = 0; t < n; ++t) ho[t] = hv[perm[t]];
+        HIPCHK(hipMemcpy(vals, ho.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
         out->nnodes = nw;
     }
+    HIPCHK(hipMemcpy(out->nodes, hn.data(), sizeof(uint32_t) * hn.size(), hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_tri_reorder, dim3((n + TRI_PAD + TB - 1) / TB), dim3(TB), 0, st, pos, vals, n, out->tri);
+    HIPCHK(hipGetLastError());
     out->depth = depth;
     HIPCHK(hipStreamSynchronize(st));
     // Host validation of the tree before any kernel traverses it: every
     // internal reference in range, every leaf range inside the triangle
     // array, every triangle in exactly one leaf, depth as measured.
     {
-        std::vector<float> hn((size_t)NF * out->nnodes);
-        HIPCHK(hipMemcpy(hn.data(), out->nodes, sizeof(float) * hn.size(), hipMemcpyDeviceToHost));
         std::vector<unsigned char> seen(n, 0);
         std::vector<int> stackv{0};
         std::vector<int> dep{1};
@@ -710,18 +767,28 @@ int build_bvh(const float* pos, int n, int width, bool sah, hipStream_t st, BvhR
             if (nd < 0 || nd >= out->nnodes || visited[nd]) { ok = false; break; }
             visited[nd] = 1;
             maxd = d > maxd ? d : maxd;
-            const uint32_t* cref = reinterpret_cast<const uint32_t*>(hn.data() + (size_t)nd * NF + 6 * width);
+            const uint32_t* w = hn.data() + (size_t)nd * NF;
+            const unsigned char* meta = reinterpret_cast<const unsigned char*>(w + 6);
+            const unsigned char* planes = reinterpret_cast<const unsigned char*>(w + NODE_PLANES(width));
             for (int k = 0; k < width; ++k) {
-                uint32_t r = cref[k];
-                if (r == EMPTY_CHILD) continue;
-                if (r & LEAF_BIT) {
-                    int start = (int)((r & ~LEAF_BIT) >> 3), cnt = (int)(r & 7u) + 1;
-                    if (start < 0 || start + cnt > n) { ok = false; break; }
-                    for (int t = start; t < start + cnt; ++t) {
+                const uint32_t o = meta[k] & 0x7fu;
+                const bool leaf = (meta[k] & NODE_LEAF) != 0, after_leaf = k > 0 && (meta[k - 1] & NODE_LEAF) != 0;
+                if (leaf && k > 0 && !after_leaf) { ok = false; break; }  // leaves come first
+                const long long start = (long long)w[5] + (after_leaf ? meta[k - 1] & 0x7fu : 0u);
+                if (planes[k] > planes[width + k]) {  // unused slot
+                    if (k == 0 || (leaf ? (long long)w[5] + o != start + 1 || start >= n + TRI_PAD : meta[k] != meta[k - 1])) ok = false;
+                    continue;
+                }
+                if (leaf) {
+                    const long long cnt = (long long)w[5] + o - start;
+                    if (cnt < 1 || cnt > DP_LEAF_MAX || start + cnt > n) { ok = false; break; }
+                    for (long long t = start; t < start + cnt; ++t) {
                         if (seen[t]) ok = false;
                         seen[t] = 1;
                     }
                 } else {
+                    const long long r = (long long)w[4] + o;
+                    if (r >= out->nnodes) { ok = false; break; }
                     stackv.push_back((int)r);
                     dep.push_back(d + 1);
                 }

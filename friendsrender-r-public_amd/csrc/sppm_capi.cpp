@@ -1167,8 +1167,14 @@ static TraceSpill trace_spill(const sppm_ctx* c) {
     return sp;
 }
 // the eye pass's own spill area: in a full pass it runs beside the photon pass
-static TraceSpill trace_spill_eye(const sppm_ctx* c) {
+// beside: in a full pass it takes 5/16 of the path-kernel grid.  Its persistent
+// waves would otherwise fill every wave slot that the gather leaves free, and
+// the build's short kernels after it wait for them (a sort pass took 1.5 ms):
+// 4M photons at 1024^2 (caustics, 8 passes) 124.5 ms against 135.5 with the
+// whole grid, the full-material workload 138.5 against 139.2 (32 passes).
+static TraceSpill trace_spill_eye(const sppm_ctx* c, bool beside) {
     TraceSpill sp = c->scene.trace_spill_eye();
+    if (beside) sp.blocks = sp.blocks * 5 / 16 > 0 ? sp.blocks * 5 / 16 : 1;
     if (c->tuned_blocks > 0 && c->tuned_blocks < sp.blocks) sp.blocks = c->tuned_blocks;
     return sp;
 }
@@ -1282,7 +1288,7 @@ static int words_generate_upto(sppm_ctx* c, long long k) {
     return SPPM_OK;
 }
 // Eye pass on stream st with the next camera word block.
-static int do_eye(sppm_ctx* c, int step, hipStream_t st, Timer* t) {
+static int do_eye(sppm_ctx* c, int step, hipStream_t st, Timer* t, bool beside = false) {
     fill_fixed_sample(c, step);
     const bool uni = c->cam.sampler == SPPM_SAMPLER_UNIFORM;
     const long long u = c->words_used;
@@ -1293,7 +1299,7 @@ static int do_eye(sppm_ctx* c, int step, hipStream_t st, Timer* t) {
         HIPOK(hipStreamWaitEvent(st, c->ev_words[b], 0));
     }
     if (t) t->start(st);
-    launch_eye(c->scene.dev, c->camdev, c->rb.hits, step, nullptr, trace_spill_eye(c),
+    launch_eye(c->scene.dev, c->camdev, c->rb.hits, step, nullptr, trace_spill_eye(c, beside),
                c->rb.words + (size_t)b * 6 * (size_t)c->rb.np, c->rb.flags, eye_rays(c->rb), c->scene.next_path + STRIPE_INTS,
                c->params.eye_nee, st);
     if (t) t->stop(st);
@@ -1473,7 +1479,7 @@ int sppm_pass(sppm_ctx* c, sppm_pass_stats* stats) {
         HIPOK(hipEventRecord(c->ev_gfork, st));
         HIPOK(hipStreamWaitEvent(c->stream2, c->ev_gfork, 0));
     }
-    rc = do_eye(c, step, c->stream2, &c->t_eye);
+    rc = do_eye(c, step, c->stream2, &c->t_eye, true);
     if (rc) return rc;
     HIPOK(hipEventRecord(c->ev_gjoin, c->stream2));
     rc = words_generate_upto(c, c->words_used);
@@ -1561,7 +1567,7 @@ static int enqueue_pass_graph(sppm_ctx* c, hipStream_t st, hipStream_t st2) {
     HIPOK(hipEventRecord(c->ev_gfork, st));
     HIPOK(hipStreamWaitEvent(st2, c->ev_gfork, 0));
     launch_camera_words(R.cam_states, R.cam_phi, R.cam_K, R.cam_L, R.words, st2);
-    launch_eye(c->scene.dev, c->camdev, R.hits, 0, R.pass_dev, trace_spill_eye(c), R.words, R.flags, eye_rays(R),
+    launch_eye(c->scene.dev, c->camdev, R.hits, 0, R.pass_dev, trace_spill_eye(c, true), R.words, R.flags, eye_rays(R),
                c->scene.next_path + STRIPE_INTS, c->params.eye_nee, st2);
     HIPOK(hipEventRecord(c->ev_gjoin, st2));
     photon_pass(c, 0, R.pass_dev, st, false);
@@ -1639,7 +1645,7 @@ int sppm_graph_capture(sppm_ctx* c) {
     for (int b = 0; b < 2 && !rc; ++b) {
         rc = capture_on(c->stream2, &c->g_eye[b], &c->x_eye[b], [&]() {
             launch_add_i32(R.pass_dev + 2, 1, c->stream2);
-            launch_eye(c->scene.dev, c->camdev, R.hitbuf[b], 0, R.pass_dev + 2, trace_spill_eye(c), R.words + b * blk,
+            launch_eye(c->scene.dev, c->camdev, R.hitbuf[b], 0, R.pass_dev + 2, trace_spill_eye(c, true), R.words + b * blk,
                        R.flags, eye_rays(R), c->scene.next_path + STRIPE_INTS, c->params.eye_nee, c->stream2);
             return SPPM_OK;
         });

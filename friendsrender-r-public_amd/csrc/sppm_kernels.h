@@ -28,7 +28,7 @@ size_t scan_tmp_entries(int n);
 
 // ---- BVH build (sppm_bvh.hip) ---------------------------------------------
 struct BvhResult {
-    float* nodes = nullptr;  // device, nnodes * node_floats(width)
+    uint32_t* nodes = nullptr;  // device, nnodes * node_words(width)
     float4* tri = nullptr;   // device, 3 * ntri
     int nnodes = 0;
     int depth = 0;           // wide levels

@@ -11,18 +11,36 @@
 namespace sppm {
 
 // ---- closest-hit structure ------------------------------------------------
-// Wide BVH node of width W (2, 4, 8): child boxes as 6 rows of W floats
-// (min x, min y, min z, max x, max y, max z), then W child references,
-// padded to a multiple of 16 bytes.  Child reference: >= 0 internal node,
-// LEAF_BIT | (start << 3) | (count - 1) leaf range of 1-8 triangles in the
-// leaf-triangle array, EMPTY_CHILD empty slot (its box is inverted).
+// Wide BVH node of width W (2, 4, 8), its child boxes as bytes in the node's own
+// frame (after Ylitie, Karras and Laine, "Efficient incoherent ray traversal on
+// GPUs through compressed wide BVHs", HPG 2017); words of 32 bits:
+//   0-2   frame origin x, y, z (float)
+//   3     frame step of x, y, z: bits 21-30 of a float each (exponent and two
+//         bits of the mantissa), 10 bits apart
+//   4     number of the first inner child (a node's inner children are consecutive)
+//   5     first leaf triangle of its leaf children (their triangles are consecutive)
+//   6..   one byte per child, leaf children first: leaf -> NODE_LEAF | the end of
+//         its triangles, counted from word 5 (they start where the leaf before
+//         ends); inner child k of the node -> k
+//   NODE_PLANES(W)..  W bytes each: min x, max x, min y, max y, min z, max z in
+//         steps from the origin, rounded outwards, so a decoded box holds its child's
+// An unused slot has inverted planes.  A ray that rounding lets into it all the
+// same comes to no harm: its byte is that of the last inner child, or of a leaf of
+// the triangle after the node's (the triangle array is padded for it).
+// A traversal reference is a node number, LEAF_BIT | (first triangle << 3) | (count - 1)
+// for a leaf, or EMPTY_CHILD (none).
+// An 80-byte node is 5 loads of 16 bytes a lane (224 and 14 with float boxes),
+// and the 18.9k nodes of a 203k-triangle scene take 1.5 MB of the 4 MB L2 (4.2 MB).
 constexpr uint32_t LEAF_BIT = 0x80000000u;
 constexpr uint32_t EMPTY_CHILD = 0xffffffffu;
 constexpr int TRACE_LDS = 16;  // traversal stack entries per lane kept in LDS (deeper ones spill)
 // LDS words of a 64-lane block's traversal stack: the node references, then
-// their boxes' entry distances
-constexpr int TRACE_STACK_WORDS = 2 * TRACE_LDS * 64;
-__host__ __device__ constexpr int node_floats(int W) { return ((7 * W + 3) / 4) * 4; }
+// their boxes' entry distances, then 32 words for trav_leaves
+constexpr int TRACE_STACK_WORDS = 2 * TRACE_LDS * 64 + 32;
+constexpr uint32_t NODE_LEAF = 0x80u;
+constexpr int TRI_PAD = 8;  // degenerate triangles after the last one
+__host__ __device__ constexpr int NODE_PLANES(int W) { return W == 8 ? 8 : 7; }
+__host__ __device__ constexpr int node_words(int W) { return W == 8 ? 20 : (W == 4 ? 16 : 12); }
 
 // Leaf triangle t (sorted order): 3 float4 = (v0.xyz, facet id bits),
 // (e1 = v1 - v0, 0), (e2 = v2 - v0, 0).  e1/e2 are exactly the reference's
@@ -63,7 +81,7 @@ struct DevLight {      // LightSampler::AreaLight (LightSampler.h:20-42)
 struct SceneDev {
     int width;                        // BVH width
     int nnodes;
-    const float* __restrict__ nodes;  // nnodes * node_floats(width)
+    const uint32_t* __restrict__ nodes;  // nnodes * node_words(width)
     int ntri;
     const float4* __restrict__ tri;   // 3 * ntri
     int nfacets;

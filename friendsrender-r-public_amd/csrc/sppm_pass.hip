@@ -169,48 +169,88 @@ __global__ void __launch_bounds__(CAMW_JUMP_THREADS) k_camw_jump_multi(const Cam
     camw_jump(J.states + (size_t)J.K * 624, J.phi, J.states, (int)blockIdx.x - kstart[s], ring);
 }
 
-// Persistent photon pass: each lane traces one path at a time; when at least
-// PHOTON_REGEN lanes of a wave have finished their paths, the wave claims the
-// next path indices from the striped path counters (one atomic per claim),
-// so lanes do not idle behind the longest path of their wave.  A path's result depends
-// only on its index, not on the lane or order that traces it.  Every wave
-// exits once the counter has passed N and its lanes are done.
+// Persistent photon pass.  A wave claims path indices from the striped path
+// counters, PHOTON_CLAIM at a time, and makes the expensive word of each
+// stream's state for all of them at once (mt_word397, one path per lane, kept
+// in LDS); its lanes then take paths from that pool one by one.  The wave
+// traces its lanes' rays together until a share of them is done, shades
+// those, gives lanes whose path ended a new one, and goes on with the rays
+// that were left, so no lane waits for the longest ray or the longest path of
+// its wave.  A path's result depends only on its index, not on the lane or
+// order that traces it.  Every wave exits once the counters have passed N and
+// its lanes are done.  128 registers, 4 waves per SIMD: 3 or 5 waves are as fast
+// in the overlapped pass (137 to 138 ms for 32 passes of the full-material
+// workload, 1 % between runs).
 // The photon paths [0, N) of one scene, traced by the calling wave until the
 // scene's counter is exhausted and the wave's lanes are done.
+constexpr int PHOTON_CLAIM = 64;  // paths a wave claims at once, at most
+// Lanes without a path before the wave starts new ones (an emission costs the
+// wave as much for one lane as for all).
+constexpr int PHOTON_START = 16;
 template <int W, bool GUIDED>
 __device__ __forceinline__ void photon_paths(const SceneDev& S, const SlotsDev& slots, int N, int step,
-                                             int* __restrict__ next_path, const GuideEmit& G, const TraceStack& ts,
-                                             uint32_t& ovf, uint32_t& fl, uint32_t& nray, uint32_t& ntie) {
+                                             int* __restrict__ next_path, int claim, const GuideEmit& G,
+                                             const TraceStack& ts, uint32_t* __restrict__ pool, uint32_t& ovf,
+                                             uint32_t& fl, uint32_t& nray, uint32_t& ntie) {
     const int lane = threadIdx.x;
     const unsigned long long below = (1ull << lane) - 1ull;
     PhotonPath P;
+    RayTrav R;
+    R.ref = EMPTY_CHILD;
     bool alive = false, exhausted = false;
+    int first = 0, have = 0, used = 0;  // the pool: paths first + [used, have)
     StripeCursor cur = stripe_start();
     for (;;) {
-        const unsigned long long idle = __ballot(!alive);
-        const int nidle = __popcll(idle);
-        if (!exhausted && nidle >= PHOTON_REGEN) {
-            int first = 0;
-            const int got = stripe_claim(next_path, N, cur, nidle, &first);
-            if (got == 0) exhausted = true;
-            if (!alive) {
-                const int r = __popcll(idle & below);
-                if (r < got) {
-                    const int i = first + r;
-                    if constexpr (GUIDED) photon_start_guided(S, slots, G, N, step, i, P, &ovf);
-                    else photon_start(S, slots, N, step, i, P, &ovf);
-                    alive = true;
-                }
+        // shade the rays that are done; next: the lane has a ray to begin
+        bool next = false;
+        if (alive && R.ref == EMPTY_CHILD) {
+            HitRec h;
+            ++nray;
+            if (trav_hit(S, P.cur_org, P.cur_dir, R, h)) {
+                ntie += h.tie ? 1u : 0u;
+                next = photon_shade(S, slots, P, h, &ovf, &fl) && photon_pretrace(P);
             }
+            if (!next) photon_finish(slots, P);
+            alive = next;
         }
-        if (__ballot(alive) == 0ull) {
+        // new paths for the idle lanes
+        for (;;) {
+            const unsigned long long idle = __ballot(!alive);
+            const int nidle = __popcll(idle);
+            if (nidle < PHOTON_START) break;
+            if (used == have) {
+                if (exhausted) break;
+                have = stripe_claim(next_path, N, cur, claim, &first);
+                used = 0;
+                if (have == 0) {
+                    exhausted = true;
+                    break;
+                }
+                __builtin_amdgcn_wave_barrier();
+                if (lane < have) pool[lane] = mt_word397(photon_seed(N, step, first + lane));
+                __builtin_amdgcn_wave_barrier();
+            }
+            const int take = min(nidle, have - used);
+            const int r = __popcll(idle & below);
+            if (!alive && r < take) {
+                const int i = first + used + r;
+                const uint32_t w397 = pool[used + r];
+                if constexpr (GUIDED) photon_start_guided(S, slots, G, N, step, i, w397, P, &ovf);
+                else photon_start(S, slots, N, step, i, w397, P, &ovf);
+                alive = next = photon_pretrace(P);
+                if (!next) photon_finish(slots, P);
+            }
+            used += take;
+        }
+        const int live = __popcll(__ballot(alive));
+        if (live == 0) {
             if (exhausted) break;
             continue;
         }
-        if (alive && !photon_bounce<W>(S, slots, P, ts, &ovf, &fl, nray, ntie)) {
-            photon_finish(slots, P);
-            alive = false;
-        }
+        if (next) trav_begin(R);
+        // until half of the wave's rays are done (a quarter: 20 % slower, its shading
+        // steps serve too few lanes; three quarters or all: the long rays hold too many)
+        trav_run<W, true>(S, P.cur_org, P.cur_dir, SPPM_RAY_OFFSET, ts, live - max(1, live / 2), R, &fl);
     }
 }
 
@@ -218,15 +258,16 @@ template <int W, bool GUIDED>
 __global__ void __launch_bounds__(PATH_BLOCK, PATH_WAVES_PER_SIMD) k_photon(SceneDev S, SlotsDev slots, int N, int step_arg,
                                                        const int* __restrict__ step_dev, int cap,
                                                        uint32_t* __restrict__ spill, int* __restrict__ next_path,
-                                                       GuideEmit G, uint32_t* __restrict__ flags,
+                                                       int claim, GuideEmit G, uint32_t* __restrict__ flags,
                                                        unsigned long long* __restrict__ rays) {
     // the pass step comes from the device pass counter when the pass is replayed from a graph
     const int step = step_dev ? *step_dev + 1 : step_arg;
     __shared__ uint32_t stk[TRACE_STACK_WORDS];
+    __shared__ uint32_t pool[PHOTON_CLAIM];
     const int lane = threadIdx.x;
-    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap};
+    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap, stk + 2 * TRACE_LDS * 64};
     uint32_t ovf = 0, fl = 0, nray = 0, ntie = 0;
-    photon_paths<W, GUIDED>(S, slots, N, step, next_path, G, ts, ovf, fl, nray, ntie);
+    photon_paths<W, GUIDED>(S, slots, N, step, next_path, claim, G, ts, pool, ovf, fl, nray, ntie);
     if (ovf) fl |= 2u;
     if (fl) atomicOr(flags, fl);
     add_wave_count(rays, nray);
@@ -261,8 +302,9 @@ __global__ void __launch_bounds__(PATH_BLOCK, PATH_WAVES_PER_SIMD) k_photon_mult
                                                                                 const int* __restrict__ bstart, int cap,
                                                                                 uint32_t* __restrict__ spill) {
     __shared__ uint32_t stk[TRACE_STACK_WORDS];
+    __shared__ uint32_t pool[PHOTON_CLAIM];
     const int lane = threadIdx.x;
-    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap};
+    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap, stk + 2 * TRACE_LDS * 64};
     const int home = home_scene(bstart, njobs);
     for (int k = 0; k < njobs; ++k) {
         const int s = __builtin_amdgcn_readfirstlane(home + k < njobs ? home + k : home + k - njobs);
@@ -270,7 +312,7 @@ __global__ void __launch_bounds__(PATH_BLOCK, PATH_WAVES_PER_SIMD) k_photon_mult
         if (scene_done(J.next_path)) continue;
         const int step = J.step_dev ? *J.step_dev + 1 : J.step;
         uint32_t ovf = 0, fl = 0, nray = 0, ntie = 0;
-        photon_paths<W, GUIDED>(J.S, J.slots, J.N, step, J.next_path, J.G, ts, ovf, fl, nray, ntie);
+        photon_paths<W, GUIDED>(J.S, J.slots, J.N, step, J.next_path, PHOTON_CLAIM, J.G, ts, pool, ovf, fl, nray, ntie);
         scene_mark_done(J.next_path);
         if (ovf) fl |= 2u;
         if (fl) atomicOr(J.flags, fl);
@@ -503,6 +545,26 @@ __device__ __forceinline__ f3 ibl_color(const SceneDev& S, f3 dir) {
 // does.  The reference recurses; this loops, passing at most OCC_LAYERS
 // surfaces (flag bit 2 beyond, counted as occluded).
 constexpr int OCC_LAYERS = 256;
+// The surface hit by ray (o, d): does it end the ray?  Otherwise the ray's rest.
+__device__ __forceinline__ bool occluder(const SceneDev& S, const HitRec& h, f3& o, f3& d, float& mn, float& mx,
+                                         float transl) {
+    const DevAttr& a = S.attrs[S.facet_attr[h.facet]];
+    if (a.tex_albedo < 0) return true;
+    const float2* tv = S.facet_uv + 3 * (size_t)h.facet;
+    const float2 t0 = tv[0], t1 = tv[1], t2 = tv[2];
+    const float uvx = ((t1.x - t0.x) * h.u + (t2.x - t0.x) * h.v) + t0.x;
+    const float uvy = ((t1.y - t0.y) * h.u + (t2.y - t0.y) * h.v) + t0.y;
+    const TexDesc td = S.tex[a.tex_albedo];
+    const float4 c = tex_bilinear(S.texels + td.offset, td.width, td.height, uvx, uvy);
+    const float tr = (float)(1.0 - (double)c.w);
+    if (!(tr > transl)) return true;
+    const float dist = h.t + SPPM_RAY_OFFSET;
+    o = o + d * dist;
+    d = normalized(d);
+    mn = fmaxf(mn - dist, SPPM_RAY_OFFSET);
+    mx = mx - dist;
+    return false;
+}
 template <int W>
 __device__ __forceinline__ bool occluded_ray(const SceneDev& S, f3 o, f3 d, float mn, float mx, float transl,
                                              const TraceStack& ts, uint32_t& fl) {
@@ -513,33 +575,43 @@ __device__ __forceinline__ bool occluded_ray(const SceneDev& S, f3 o, f3 d, floa
         }
         HitRec h;
         if (!closest_hit<W>(S, o, d, mn, ts, h, &fl) || !((double)h.t < (double)mx - 1e-10)) return false;
-        const DevAttr& a = S.attrs[S.facet_attr[h.facet]];
-        if (a.tex_albedo < 0) return true;
-        const float2* tv = S.facet_uv + 3 * (size_t)h.facet;
-        const float2 t0 = tv[0], t1 = tv[1], t2 = tv[2];
-        const float uvx = ((t1.x - t0.x) * h.u + (t2.x - t0.x) * h.v) + t0.x;
-        const float uvy = ((t1.y - t0.y) * h.u + (t2.y - t0.y) * h.v) + t0.y;
-        const TexDesc td = S.tex[a.tex_albedo];
-        const float4 c = tex_bilinear(S.texels + td.offset, td.width, td.height, uvx, uvy);
-        const float tr = (float)(1.0 - (double)c.w);
-        if (!(tr > transl)) return true;
-        const float dist = h.t + SPPM_RAY_OFFSET;
-        o = o + d * dist;
-        d = normalized(d);
-        mn = fmaxf(mn - dist, SPPM_RAY_OFFSET);
-        mx = mx - dist;
+        if (occluder(S, h, o, d, mn, mx, transl)) return true;
     }
+}
+// The same for a whole wave; on: the lane has a ray.
+template <int W>
+__device__ __forceinline__ bool occluded_wave(const SceneDev& S, bool on, f3 o, f3 d, float mn, float mx, float transl,
+                                              const TraceStack& ts, uint32_t& fl) {
+    bool occ = false;
+    for (int layer = 0; __ballot(on) != 0ull; ++layer) {
+        if (layer == OCC_LAYERS) {
+            if (on) fl |= 4u;
+            return occ || on;
+        }
+        HitRec h;
+        const bool hit = closest_hit_wave<W>(S, on, o, d, mn, ts, h, &fl);
+        if (on) {
+            on = hit && (double)h.t < (double)mx - 1e-10;
+            if (on && occluder(S, h, o, d, mn, mx, transl)) {
+                occ = true;
+                on = false;
+            }
+        }
+    }
+    return occ;
 }
 
 // NEE: the compiled-out next-event estimation of getHitpointInfo
 // (SPPM.cpp:144-168, 187-229); keep: keep what it estimates (SPPM_NEE_KEEP).
 template <int W, bool NEE>
-__device__ __forceinline__ void eye_path(const SceneDev& S, const CamDev& C, const HitDev& H, int step, int i,
+__device__ __forceinline__ void eye_path(const SceneDev& S, const CamDev& C, const HitDev& H, int step, int i, bool on,
                                          const uint32_t* __restrict__ words, const TraceStack& ts, uint32_t& fl,
                                          bool keep, uint32_t& nray, uint32_t& ntie) {
+    const bool mine = on;
     uint32_t ovf = 0;
     MTCursor m;
-    mt_seed(m, (uint32_t)i + (uint32_t)C.W * (uint32_t)C.H * (uint32_t)step);
+    const uint32_t seed = (uint32_t)i + (uint32_t)C.W * (uint32_t)C.H * (uint32_t)step;
+    mt_seed(m, seed, mt_word397(seed));
     const int w = i % C.W, hh = i / C.W;
     const float u = (float)w / (float)C.W, v = (float)hh / (float)C.H;
     f3 smp;
@@ -561,9 +633,20 @@ __device__ __forceinline__ void eye_path(const SceneDev& S, const CamDev& C, con
     f3 T = mk(1.0f, 1.0f, 1.0f);
     float PDF = 1.0f;
     int depth = 0;
-    int type = 0, facet = -1, kind = 0;
-    f3 hpos = mk(0, 0, 0), hout = mk(0, 1, 0), hw = mk(1, 1, 1), hn = mk(0, 0, 0);
-    float hidx = 1.0f, hrough = 1.0f, habs = 1.0f, hrefl = 1.0f;
+    int type = 0;
+    // The hit point is stored where it is made, not carried to the path's end
+    // (a score of registers, spilled across every trace): createHitpoints'
+    // PixelWeight /= pdf (SPPM.cpp:346-347) is all that follows.
+    auto store = [&](f3 pos, int ty, f3 n, float idx, f3 out, float rough, f3 w, float refl, int kd, int fct, float ab) {
+        w = w / campdf;
+        if (ty == 1 && (!isfinite(w.x) || !isfinite(w.y) || !isfinite(w.z))) fl |= 32u;
+        H.pos[i] = make_float4(pos.x, pos.y, pos.z, (float)ty);
+        H.nrm[i] = make_float4(n.x, n.y, n.z, idx);
+        H.out[i] = make_float4(out.x, out.y, out.z, rough);
+        H.weight[i] = make_float4(w.x, w.y, w.z, refl);
+        H.mat[i] = make_int2(kd, fct);
+        H.absorb[i] = ab;
+    };
     f3 direct = mk(0.0f, 0.0f, 0.0f);
     const bool ibl = S.ibl_tex >= 0;
     // TraceParam::PrevGmt (position, IfDeltaSurface) and pdf_prevDir (SPPM.h:78-80)
@@ -571,21 +654,27 @@ __device__ __forceinline__ void eye_path(const SceneDev& S, const CamDev& C, con
     float pdf_prev = 0.0f;
     bool prev_delta = false;
     for (;;) {
-        if (depth > 6) break;
-        else if (depth > 4) {
-            float rus = (float)exp((double)(4 - depth));
-            if (real1(m, &ovf) > (double)rus) break;
-            PDF *= rus;
+        if (on) {
+            if (depth > 6) on = false;
+            else if (depth > 4) {
+                float rus = (float)exp((double)(4 - depth));
+                if (real1(m, &ovf) > (double)rus) on = false;
+                else PDF *= rus;
+            }
         }
+        if (__ballot(on) == 0ull) break;
+        // the wave traces its lanes' rays together; then each lane goes on by itself
         HitRec h;
+        const bool got = closest_hit_wave<W>(S, on, cur_org, cur_dir, SPPM_RAY_OFFSET, ts, h, &fl);
+        if (!on) continue;
         ++nray;
-        const bool got = closest_hit<W>(S, cur_org, cur_dir, SPPM_RAY_OFFSET, ts, h, &fl);
-        ntie += h.tie ? 1u : 0u;
+        ntie += got && h.tie ? 1u : 0u;
+        on = [&]() -> bool {
         if (!got) {
             // escape: the environment's colour (SPPM.cpp:290-300)
             if (ibl) direct = direct + (ibl_color(S, cur_dir) * T) / PDF;
             if (type == 0) type = 2;
-            break;
+            return false;
         }
         Geom g;
         calc_geometry(S, h, g);
@@ -594,7 +683,7 @@ __device__ __forceinline__ void eye_path(const SceneDev& S, const CamDev& C, con
         if (g.transl > 0.5f) {
             T = T * g.transl;
             cur_org = g.pos + cur_dir * SPPM_RAY_OFFSET;
-            continue;
+            return true;
         }
         if (NEE && norm2(g.radiance) > LO_1EM6) {  // (double)norm2 > 1e-6
             // an emitter ends the path; before the hit point its radiance is
@@ -618,24 +707,15 @@ __device__ __forceinline__ void eye_path(const SceneDev& S, const CamDev& C, con
                 direct = direct + (((g.albedo * mis) * g.radiance) * T) / PDF;
                 if (keep && type == 0) type = 2;
             }
-            break;
+            return false;
         }
         if (g.is_sppm && type != 1) {  // makeHitPoint (SPPM.cpp:79-96, 171-174)
             if (!(NEE && keep)) direct = mk(0.0f, 0.0f, 0.0f);  // the new HitPoint's DirectLight
             type = 1;
-            facet = h.facet;
-            hpos = g.pos;
-            hout = -cur_dir;
-            hw = T / PDF;
-            hn = Nf;
-            kind = g.kind;
-            hidx = g.index;
-            hrough = g.rough;
-            habs = g.absorb;
-            hrefl = g.refl;
+            store(g.pos, 1, Nf, g.index, -cur_dir, g.rough, T / PDF, g.refl, g.kind, h.facet, g.absorb);
             // the path goes on after its hit point only to reach the
             // environment; without one nothing later changes the hit point
-            if (!ibl) break;
+            if (!ibl) return false;
         }
         float Ii, Io = 1.0f;
         if (near1(cur_index)) { Ii = 1.0f; Io = g.index; }
@@ -676,9 +756,9 @@ __device__ __forceinline__ void eye_path(const SceneDev& S, const CamDev& C, con
         }
         float pdf_s = 1.0f;
         next_dir = surf_sample(g.kind, fp, m, &ovf, &pdf_s);
-        if (!rutil_valid_dir(next_dir)) break;
+        if (!rutil_valid_dir(next_dir)) return false;
         if (g.opaque) {
-            if (dot(next_dir, Nf) < HI_1EM6) break;  // (double)dot < 1e-6
+            if (dot(next_dir, Nf) < HI_1EM6) return false;  // (double)dot < 1e-6
         } else {
             next_index = !(dot(next_dir, Nf) < 0.0f) ? cur_index : Io;
         }
@@ -688,8 +768,8 @@ __device__ __forceinline__ void eye_path(const SceneDev& S, const CamDev& C, con
         next_org = next_org + outN * SPPM_RAY_OFFSET;
         float brdf = surf_brdf(g.kind, fp);
         float cs = smax(0.0f, smin(1.0f, dot(next_dir, outN)));
-        if (brdf < HI_1EM8) break;  // (double)brdf < 1e-8
-        if (pdf_s < 0) break;
+        if (brdf < HI_1EM8) return false;  // (double)brdf < 1e-8
+        if (pdf_s < 0) return false;
         T = T * ((g.albedo * cs) * brdf);
         PDF *= pdf_s;
         if (NEE) {
@@ -701,39 +781,37 @@ __device__ __forceinline__ void eye_path(const SceneDev& S, const CamDev& C, con
         cur_dir = next_dir;
         cur_index = next_index;
         ++depth;
+        return true;
+        }();
     }
-    hw = hw / campdf;  // createHitpoints: PixelWeight /= pdf, DirectLight /= pdf (SPPM.cpp:346-347)
+    if (!mine) return;
+    if (type != 1)
+        store(mk(0, 0, 0), type, mk(0, 0, 0), 1.0f, mk(0, 1, 0), 1.0f, mk(1, 1, 1), 1.0f, 0, -1, 1.0f);
     if (ibl || NEE) {
-        direct = direct / campdf;
+        direct = direct / campdf;  // DirectLight /= pdf
         H.direct[i] = make_float4(direct.x, direct.y, direct.z, 0.0f);
     }
-    if (type == 1 && (!isfinite(hw.x) || !isfinite(hw.y) || !isfinite(hw.z))) fl |= 32u;
-    H.pos[i] = make_float4(hpos.x, hpos.y, hpos.z, (float)type);
-    H.nrm[i] = make_float4(hn.x, hn.y, hn.z, hidx);
-    H.out[i] = make_float4(hout.x, hout.y, hout.z, hrough);
-    H.weight[i] = make_float4(hw.x, hw.y, hw.z, hrefl);
-    H.mat[i] = make_int2(kind, facet);
-    H.absorb[i] = habs;
     if (ovf) fl |= 2u;
 }
 
-// Eye pass: persistent waves take 64 consecutive pixels at a time from a
+// Eye pass: persistent waves take up to 64 consecutive pixels at a time from a
 // counter (zeroed before the launch), so waves whose pixels have long paths
 // (glass, mirrors) do not hold back the others; a pixel's result does not
 // depend on the wave that traces it.
-// The pixels of one scene, 64 at a time, until its counter is exhausted.
+// The pixels of one scene, `claim` at a time, until its counter is exhausted.
 template <int W, bool NEE>
 __device__ __forceinline__ void eye_pixels(const SceneDev& S, const CamDev& C, const HitDev& H, int step,
-                                           const uint32_t* __restrict__ words, int* __restrict__ queue, bool keep,
+                                           const uint32_t* __restrict__ words, int* __restrict__ queue, int claim, bool keep,
                                            const TraceStack& ts, uint32_t& fl, uint32_t& nray, uint32_t& ntie) {
     const int lane = threadIdx.x;
     const int NPIX = C.W * C.H;
     StripeCursor cur = stripe_start();
     for (;;) {
         int first = 0;
-        const int got = stripe_claim(queue, NPIX, cur, 64, &first);
+        const int got = stripe_claim(queue, NPIX, cur, claim, &first);
         if (got == 0) break;
-        if ((lane & 63) < got) eye_path<W, NEE>(S, C, H, step, first + (lane & 63), words, ts, fl, keep, nray, ntie);
+        // lanes past the claim stand at its last pixel and write nothing
+        eye_path<W, NEE>(S, C, H, step, first + min(lane, got - 1), lane < got, words, ts, fl, keep, nray, ntie);
     }
 }
 
@@ -742,13 +820,14 @@ __global__ void __launch_bounds__(PATH_BLOCK, PATH_WAVES_PER_SIMD) k_eye(SceneDe
                                                     const int* __restrict__ step_dev, int cap,
                                                     uint32_t* __restrict__ spill, const uint32_t* __restrict__ words,
                                                     uint32_t* __restrict__ flags, int keep,
-                                                    unsigned long long* __restrict__ rays, int* __restrict__ queue) {
+                                                    unsigned long long* __restrict__ rays, int* __restrict__ queue,
+                                                    int claim) {
     const int step = step_dev ? *step_dev + 1 : step_arg;
     __shared__ uint32_t stk[TRACE_STACK_WORDS];
     const int lane = threadIdx.x;
-    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap};
+    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap, stk + 2 * TRACE_LDS * 64};
     uint32_t fl = 0, nray = 0, ntie = 0;
-    eye_pixels<W, NEE>(S, C, H, step, words, queue, keep != 0, ts, fl, nray, ntie);
+    eye_pixels<W, NEE>(S, C, H, step, words, queue, claim, keep != 0, ts, fl, nray, ntie);
     if (fl) atomicOr(flags, fl);
     add_wave_count(rays, nray);
     add_wave_count(rays + 2, ntie);
@@ -761,7 +840,7 @@ __global__ void __launch_bounds__(PATH_BLOCK, PATH_WAVES_PER_SIMD) k_eye_multi(c
                                                                              uint32_t* __restrict__ spill) {
     __shared__ uint32_t stk[TRACE_STACK_WORDS];
     const int lane = threadIdx.x;
-    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap};
+    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap, stk + 2 * TRACE_LDS * 64};
     const int home = home_scene(bstart, njobs);
     for (int k = 0; k < njobs; ++k) {
         const int s = __builtin_amdgcn_readfirstlane(home + k < njobs ? home + k : home + k - njobs);
@@ -769,7 +848,7 @@ __global__ void __launch_bounds__(PATH_BLOCK, PATH_WAVES_PER_SIMD) k_eye_multi(c
         if (scene_done(J.queue)) continue;
         const int step = J.step_dev ? *J.step_dev + 1 : J.step;
         uint32_t fl = 0, nray = 0, ntie = 0;
-        eye_pixels<W, NEE>(J.S, J.C, J.H, step, J.words, J.queue, J.keep != 0, ts, fl, nray, ntie);
+        eye_pixels<W, NEE>(J.S, J.C, J.H, step, J.words, J.queue, 64, J.keep != 0, ts, fl, nray, ntie);
         scene_mark_done(J.queue);
         if (fl) atomicOr(J.flags, fl);
         add_wave_count(J.rays, nray);
@@ -1563,20 +1642,23 @@ __global__ void k_set_u32(uint32_t* p, uint32_t v) { *p = v; }
 // (tmin, tmax) (bvh8.h:591, 640: the MaxT test in double); a miss gives facet
 // -1, t = FLT_MAX, u = v = 0.  t, u, v may be NULL.
 template <int W>
-__global__ void __launch_bounds__(PATH_BLOCK) k_trace(SceneDev S, int n, const float* __restrict__ org,
+__global__ void __launch_bounds__(PATH_BLOCK) k_trace(SceneDev S, int n, int share, const float* __restrict__ org,
                                                       const float* __restrict__ dir, float tmin, float tmax, int cap,
                                                       uint32_t* __restrict__ spill, int* __restrict__ facet,
                                                       float* __restrict__ t, float* __restrict__ u,
                                                       float* __restrict__ v, uint32_t* __restrict__ flags) {
     __shared__ uint32_t stk[TRACE_STACK_WORDS];
     const int lane = threadIdx.x;
-    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap};
+    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap, stk + 2 * TRACE_LDS * 64};
     uint32_t fl = 0;
-    for (int i = blockIdx.x * PATH_BLOCK + lane; i < n; i += gridDim.x * PATH_BLOCK) {
+    for (int base = blockIdx.x * share; base < n; base += gridDim.x * share) {
+        const bool on = lane < share && base + lane < n;
+        const int i = on ? base + lane : base;
         HitRec h;
         f3 o = mk(org[3 * i], org[3 * i + 1], org[3 * i + 2]);
         f3 d = mk(dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]);
-        bool hit = closest_hit<W>(S, o, d, tmin, ts, h, &fl);
+        bool hit = closest_hit_wave<W>(S, on, o, d, tmin, ts, h, &fl);
+        if (!on) continue;
         hit = hit && (double)h.t < (double)tmax - 1e-10;
         facet[i] = hit ? h.facet : -1;
         if (t) t[i] = hit ? h.t : 3.40282347e38f;
@@ -1588,19 +1670,22 @@ __global__ void __launch_bounds__(PATH_BLOCK) k_trace(SceneDev S, int n, const f
 
 // Scene::IsOccluded for a batch of rays (MaxDist per ray).
 template <int W>
-__global__ void __launch_bounds__(PATH_BLOCK) k_occluded(SceneDev S, int n, const float* __restrict__ org,
+__global__ void __launch_bounds__(PATH_BLOCK) k_occluded(SceneDev S, int n, int share, const float* __restrict__ org,
                                                          const float* __restrict__ dir, float tmin,
                                                          const float* __restrict__ tmax, float transl, int cap,
                                                          uint32_t* __restrict__ spill,
                                                          int* __restrict__ occluded, uint32_t* __restrict__ flags) {
     __shared__ uint32_t stk[TRACE_STACK_WORDS];
     const int lane = threadIdx.x;
-    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap};
+    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap, stk + 2 * TRACE_LDS * 64};
     uint32_t fl = 0;
-    for (int i = blockIdx.x * PATH_BLOCK + lane; i < n; i += gridDim.x * PATH_BLOCK) {
+    for (int base = blockIdx.x * share; base < n; base += gridDim.x * share) {
+        const bool on = lane < share && base + lane < n;
+        const int i = on ? base + lane : base;
         const f3 o = mk(org[3 * i], org[3 * i + 1], org[3 * i + 2]);
         const f3 d = mk(dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]);
-        occluded[i] = occluded_ray<W>(S, o, d, tmin, tmax[i], transl, ts, fl) ? 1 : 0;
+        const bool occ = occluded_wave<W>(S, on, o, d, tmin, tmax[i], transl, ts, fl);
+        if (on) occluded[i] = occ ? 1 : 0;
     }
     if (fl) atomicOr(flags, fl);
 }
@@ -1632,14 +1717,28 @@ void launch_camera_words_multi(const CamJob* jobs, const int* kstart, int njobs,
     hipLaunchKernelGGL(k_camw_jump_multi, dim3(nseg), dim3(CAMW_JUMP_THREADS), 0, st, jobs, kstart, njobs);
 }
 
+// Items (paths, pixels, rays) a wave takes at a time: as many as there are for
+// each of WAVE_SHARE_WAVES waves (one for every SIMD of the chip), so that few
+// items spread over all of them instead of filling the lanes of a few, whose
+// paths then wait for each other: a render of 5k photons and 64^2 pixels takes
+// 4.1 ms with one to five items a wave, 4.8 with 64.  With more waves than
+// that the lanes left empty cost more than the waiting: 100k photons and 256^2
+// pixels 17.3 ms with 64 items a wave, 18.4 when spread over 4096 waves.
+constexpr int WAVE_SHARE_WAVES = 1024;
+static int wave_share(long long items) {
+    const long long s = (items + WAVE_SHARE_WAVES - 1) / WAVE_SHARE_WAVES;
+    return (int)(s < 1 ? 1 : s > 64 ? 64 : s);
+}
+
 void launch_photon(const SceneDev& S, const SlotsDev& slots, int N, int step, const int* step_dev,
                    const TraceSpill& sp, int* next_path, const GuideEmit* guide, uint32_t* flags,
                    unsigned long long* rays, hipStream_t st) {
     hipLaunchKernelGGL(k_zero_i32, dim3(STRIPE_INTS / 256), dim3(256), 0, st, next_path, STRIPE_INTS);
     dim3 g(sp.blocks), b(PATH_BLOCK);
     const GuideEmit G = guide ? *guide : GuideEmit{};
+    const int claim = wave_share(N);
 #define SPPM_PHOTON(WW, GG) \
-    hipLaunchKernelGGL((k_photon<WW, GG>), g, b, 0, st, S, slots, N, step, step_dev, sp.cap, sp.buf, next_path, G, \
+    hipLaunchKernelGGL((k_photon<WW, GG>), g, b, 0, st, S, slots, N, step, step_dev, sp.cap, sp.buf, next_path, claim, G, \
                        flags, rays)
     if (guide) {
         if (S.width == 2) SPPM_PHOTON(2, true);
@@ -1659,15 +1758,16 @@ static void launch_eye_t(const SceneDev& S, const CamDev& C, const HitDev& H, in
                          int* queue, int keep, hipStream_t st) {
     hipLaunchKernelGGL(k_zero_i32, dim3(STRIPE_INTS / 256), dim3(256), 0, st, queue, STRIPE_INTS);
     dim3 g(sp.blocks), b(PATH_BLOCK);
+    const int claim = wave_share((long long)C.W * C.H);
     if (S.width == 2)
         hipLaunchKernelGGL((k_eye<2, NEE>), g, b, 0, st, S, C, H, step, step_dev, sp.cap, sp.buf, words, flags, keep,
-                           rays, queue);
+                           rays, queue, claim);
     else if (S.width == 4)
         hipLaunchKernelGGL((k_eye<4, NEE>), g, b, 0, st, S, C, H, step, step_dev, sp.cap, sp.buf, words, flags, keep,
-                           rays, queue);
+                           rays, queue, claim);
     else
         hipLaunchKernelGGL((k_eye<8, NEE>), g, b, 0, st, S, C, H, step, step_dev, sp.cap, sp.buf, words, flags, keep,
-                           rays, queue);
+                           rays, queue, claim);
 }
 void launch_eye(const SceneDev& S, const CamDev& C, const HitDev& H, int step, const int* step_dev,
                 const TraceSpill& sp, const uint32_t* words, uint32_t* flags, unsigned long long* rays, int* queue,
@@ -1688,8 +1788,9 @@ void launch_zero_i32(int* p, int n, hipStream_t st) {
 void launch_trace(const SceneDev& S, int n, const float* org, const float* dir, float tmin, float tmax,
                   const TraceSpill& sp, int* facet, float* t, float* u, float* v, uint32_t* flags, hipStream_t st) {
     dim3 g(sp.blocks), b(PATH_BLOCK);
+    const int share = wave_share(n);
 #define SPPM_TRACE(WW) \
-    hipLaunchKernelGGL(k_trace<WW>, g, b, 0, st, S, n, org, dir, tmin, tmax, sp.cap, sp.buf, facet, t, u, v, flags)
+    hipLaunchKernelGGL(k_trace<WW>, g, b, 0, st, S, n, share, org, dir, tmin, tmax, sp.cap, sp.buf, facet, t, u, v, flags)
     if (S.width == 2) SPPM_TRACE(2);
     else if (S.width == 4) SPPM_TRACE(4);
     else SPPM_TRACE(8);
@@ -1700,12 +1801,13 @@ void launch_occluded(const SceneDev& S, int n, const float* org, const float* di
                      float transl,
                      const TraceSpill& sp, int* occluded, uint32_t* flags, hipStream_t st) {
     dim3 g(sp.blocks), b(PATH_BLOCK);
+    const int share = wave_share(n);
     if (S.width == 2)
-        hipLaunchKernelGGL(k_occluded<2>, g, b, 0, st, S, n, org, dir, tmin, tmax, transl, sp.cap, sp.buf, occluded, flags);
+        hipLaunchKernelGGL(k_occluded<2>, g, b, 0, st, S, n, share, org, dir, tmin, tmax, transl, sp.cap, sp.buf, occluded, flags);
     else if (S.width == 4)
-        hipLaunchKernelGGL(k_occluded<4>, g, b, 0, st, S, n, org, dir, tmin, tmax, transl, sp.cap, sp.buf, occluded, flags);
+        hipLaunchKernelGGL(k_occluded<4>, g, b, 0, st, S, n, share, org, dir, tmin, tmax, transl, sp.cap, sp.buf, occluded, flags);
     else
-        hipLaunchKernelGGL(k_occluded<8>, g, b, 0, st, S, n, org, dir, tmin, tmax, transl, sp.cap, sp.buf, occluded, flags);
+        hipLaunchKernelGGL(k_occluded<8>, g, b, 0, st, S, n, share, org, dir, tmin, tmax, transl, sp.cap, sp.buf, occluded, flags);
 }
 
 void launch_photon_stage(const SlotsDev& slots, const int* off, const StagedPhotons& sp, hipStream_t st) {

@@ -78,13 +78,18 @@ __device__ __forceinline__ float light_pick_pdf(const SceneDev& S, const DevLigh
     return L.flux_norm / S.lpick_avg / (float)S.nlights;
 }
 
+// Seed of photon path i's stream.
+__device__ __forceinline__ uint32_t photon_seed(int N, int step, int i) {
+    return (uint32_t)i + 135u + (uint32_t)step * (uint32_t)N;
+}
+
 // generateLightRay (SPPM.cpp:453-471) + the emission photon in slot 0
 // (SPPM.cpp:530-540); the first stored surface photon overwrites that slot
 // (SPPM.cpp:606), so writing it up front leaves the same slot contents.
 __device__ __forceinline__ void photon_start(const SceneDev& S, const SlotsDev& slots, int N, int step, int i,
-                                             PhotonPath& P, uint32_t* ovf) {
+                                             uint32_t word397, PhotonPath& P, uint32_t* ovf) {
     P.i = i;
-    mt_seed(P.m, (uint32_t)i + 135u + (uint32_t)step * (uint32_t)N);
+    mt_seed(P.m, photon_seed(N, step, i), word397);
     const int li = table_sample(S.lpick_prob, S.lpick_left, S.lpick_right, S.nlights, P.m, ovf);
     const DevLight& L = S.lights[li];
     f3 lpos, rad;
@@ -133,9 +138,10 @@ __device__ __forceinline__ int cdf_search(const float* __restrict__ cdf, int lo,
     return lo;
 }
 __device__ __forceinline__ void photon_start_guided(const SceneDev& S, const SlotsDev& slots, const GuideEmit& G,
-                                                    int N, int step, int i, PhotonPath& P, uint32_t* ovf) {
+                                                    int N, int step, int i, uint32_t word397, PhotonPath& P,
+                                                    uint32_t* ovf) {
     P.i = i;
-    mt_seed(P.m, (uint32_t)i + 135u + (uint32_t)step * (uint32_t)N);
+    mt_seed(P.m, photon_seed(N, step, i), word397);
     const f3 P0 = mk(G.P0[0], G.P0[1], G.P0[2]), E1 = mk(G.e1[0], G.e1[1], G.e1[2]), E2 = mk(G.e2[0], G.e2[1], G.e2[2]);
     const f3 Nn = mk(G.n[0], G.n[1], G.n[2]), T1 = mk(G.t1[0], G.t1[1], G.t1[2]), T2 = mk(G.t2[0], G.t2[1], G.t2[2]);
     const float total = G.cdf[GUIDE_CELLS - 1];

@@ -5,11 +5,25 @@
 // with identical float operations; a hit is accepted when t > MinT and
 // (t < best, or t == best and the facet id is lower): ties go to the lowest
 // facet id, so the result is independent of the tree shape and width.
-// Child boxes are padded by 0.001 like AABB::Expand (Intersect.cpp:556-575),
-// and the slab test is inclusive, so no box containing an accepted hit is
-// ever culled.  The slab distances are fma(bound, 1/d, -o/d): one FMA per
-// plane, whose rounding differs from (bound - o)/d by far less than the
-// padding (culling decides only which boxes are visited, never the hit).
+// Child boxes are padded by 0.001 like AABB::Expand (Intersect.cpp:556-575) and
+// rounded outwards to the node's byte grid, and the slab test is inclusive, so no
+// box containing an accepted hit is ever culled: the rounding of the slab
+// distances, fma(byte, step/d, (origin - o)/d), is far below the padding
+// (culling decides only which boxes are visited, never the hit).
+//
+// What bounds it: vector instructions, most of them issued for few lanes.  A
+// path wave that traced all its lanes' rays to the end, then shaded them, ran
+// with 8 of 64 lanes on average.  Hence three things.  The traversal's state can
+// be left and taken up again (RayTrav), so that a wave shades the rays that are
+// done while the others go on; the lanes of a wave take node steps and leaf
+// steps by turns (trav_run); and a leaf's triangles are spread over the lanes
+// (trav_leaves).  With the byte nodes and their one-word sort keys (about 300
+// instructions and 5 loads a node; 900, with a branch per comparator, and 14)
+// the photon pass alone went from 2.80 to 1.97 ms (1M photons, 203k triangles),
+// 11.3 to 6.0 ms (4M photons, 500k triangles of rough glass), the eye pass
+// 0.72 to 0.61 and 2.39 to 1.63 ms (1024^2), 1M rays through the 203k triangles
+// 0.62 to 0.41 ms, 20k shadow rays 0.078 to 0.053 ms.  (These photon and eye
+// times include the shading's own gains, see lobe_draw.)
 //
 // Traversal descends into the nearest intersected child and pushes the
 // others far-to-near.  The first TRACE_LDS stack entries of a lane live in
@@ -29,6 +43,7 @@ struct TraceStack {
     uint32_t* glob;  // spill area + the lane's slot; stride gstride
     int gstride;
     int cap;         // total entries
+    uint32_t* own;   // LDS of the wave: 32 words (trav_leaves)
 };
 
 struct HitRec {
@@ -40,10 +55,11 @@ struct HitRec {
 };
 
 __device__ __forceinline__ bool tri_test(const float4* __restrict__ tri, int slot, f3 org, f3 dir, float& t,
-                                         float& u, float& v) {
+                                         float& u, float& v, int& facet) {
     float4 A = tri[3 * slot + 0];
     float4 B = tri[3 * slot + 1];
     float4 C = tri[3 * slot + 2];
+    facet = __float_as_int(A.w);
     f3 p0 = mk(A.x, A.y, A.z);
     f3 e1 = mk(B.x, B.y, B.z);
     f3 e2 = mk(C.x, C.y, C.z);
@@ -63,33 +79,81 @@ __device__ __forceinline__ bool tri_test(const float4* __restrict__ tri, int slo
     return true;
 }
 
-__device__ __forceinline__ void cswap(float& da, uint32_t& ra, float& db, uint32_t& rb) {
-    // keep ascending distance: (da, ra) <= (db, rb)
-    if (db < da) {
-        float td = da; da = db; db = td;
-        uint32_t tr = ra; ra = rb; rb = tr;
-    }
+__device__ __forceinline__ void cswap(uint32_t& a, uint32_t& b) {
+    const uint32_t lo = min(a, b), hi = max(a, b);
+    a = lo;
+    b = hi;
 }
 template <int W>
-__device__ __forceinline__ void sort_children(float* d, uint32_t* r) {
+__device__ __forceinline__ void sort_keys(uint32_t* k) {
     if constexpr (W == 2) {
-        cswap(d[0], r[0], d[1], r[1]);
+        cswap(k[0], k[1]);
     } else if constexpr (W == 4) {
-        cswap(d[0], r[0], d[1], r[1]); cswap(d[2], r[2], d[3], r[3]);
-        cswap(d[0], r[0], d[2], r[2]); cswap(d[1], r[1], d[3], r[3]);
-        cswap(d[1], r[1], d[2], r[2]);
+        cswap(k[0], k[1]); cswap(k[2], k[3]);
+        cswap(k[0], k[2]); cswap(k[1], k[3]);
+        cswap(k[1], k[2]);
     } else {
         // Batcher odd-even merge sort network for 8 inputs (19 comparators)
-        cswap(d[0], r[0], d[1], r[1]); cswap(d[2], r[2], d[3], r[3]);
-        cswap(d[4], r[4], d[5], r[5]); cswap(d[6], r[6], d[7], r[7]);
-        cswap(d[0], r[0], d[2], r[2]); cswap(d[1], r[1], d[3], r[3]);
-        cswap(d[4], r[4], d[6], r[6]); cswap(d[5], r[5], d[7], r[7]);
-        cswap(d[1], r[1], d[2], r[2]); cswap(d[5], r[5], d[6], r[6]);
-        cswap(d[0], r[0], d[4], r[4]); cswap(d[1], r[1], d[5], r[5]);
-        cswap(d[2], r[2], d[6], r[6]); cswap(d[3], r[3], d[7], r[7]);
-        cswap(d[2], r[2], d[4], r[4]); cswap(d[3], r[3], d[5], r[5]);
-        cswap(d[1], r[1], d[2], r[2]); cswap(d[3], r[3], d[4], r[4]);
-        cswap(d[5], r[5], d[6], r[6]);
+        cswap(k[0], k[1]); cswap(k[2], k[3]); cswap(k[4], k[5]); cswap(k[6], k[7]);
+        cswap(k[0], k[2]); cswap(k[1], k[3]); cswap(k[4], k[6]); cswap(k[5], k[7]);
+        cswap(k[1], k[2]); cswap(k[5], k[6]);
+        cswap(k[0], k[4]); cswap(k[1], k[5]); cswap(k[2], k[6]); cswap(k[3], k[7]);
+        cswap(k[2], k[4]); cswap(k[3], k[5]);
+        cswap(k[1], k[2]); cswap(k[3], k[4]); cswap(k[5], k[6]);
+    }
+}
+
+// The ray in the frame of a node (layout: sppm_layout.h): plane q of axis a
+// is crossed at fma(q, step.a, org.a).
+struct NodeFrame {
+    f3 step, org;
+};
+__device__ __forceinline__ NodeFrame node_frame(const uint32_t* w, f3 org, f3 inv) {
+    NodeFrame f;
+    f.step.x = __uint_as_float((w[3] & 0x3ffu) << 21) * inv.x;
+    f.step.y = __uint_as_float(((w[3] >> 10) & 0x3ffu) << 21) * inv.y;
+    f.step.z = __uint_as_float((w[3] >> 20) << 21) * inv.z;
+    f.org.x = (__uint_as_float(w[0]) - org.x) * inv.x;
+    f.org.y = (__uint_as_float(w[1]) - org.y) * inv.y;
+    f.org.z = (__uint_as_float(w[2]) - org.z) * inv.z;
+    return f;
+}
+__device__ __forceinline__ float byte_f(uint32_t w, int k) { return (float)((w >> (8 * k)) & 0xffu); }
+// The planes of axis a that a ray crosses first (far: last), child c's in byte
+// c & 3 of word c >> 2; neg: the ray runs towards smaller coordinates.
+template <int W>
+__device__ __forceinline__ void node_planes(const uint32_t* w, int a, bool neg, uint32_t* near_, uint32_t* far_) {
+    const uint32_t* p = w + NODE_PLANES(W);
+    if constexpr (W == 8) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t lo = p[4 * a + h], hi = p[4 * a + 2 + h];
+            near_[h] = neg ? hi : lo;
+            far_[h] = neg ? lo : hi;
+        }
+    } else if constexpr (W == 4) {
+        const uint32_t lo = p[2 * a], hi = p[2 * a + 1];
+        near_[0] = neg ? hi : lo;
+        far_[0] = neg ? lo : hi;
+    } else {
+        const uint32_t lo = p[a], hi = p[a] >> 16;
+        near_[0] = neg ? hi : lo;
+        far_[0] = neg ? lo : hi;
+    }
+}
+// The traversal reference of the child in a slot: m its byte, p the byte of the
+// slot before (0 for the first).
+__device__ __forceinline__ uint32_t node_ref(const uint32_t* w, uint32_t m, uint32_t p) {
+    const uint32_t leaf = LEAF_BIT | ((w[5] + (p & 0x7fu)) << 3) | (((m & 0x7fu) - (p & 0x7fu) - 1u) & 7u);
+    return m & NODE_LEAF ? leaf : w[4] + (m & 0x7fu);
+}
+template <int W>
+__device__ __forceinline__ uint32_t node_child(const uint32_t* w, uint32_t slot) {
+    if constexpr (W == 8) {
+        const unsigned long long m = ((unsigned long long)w[7] << 32) | w[6];
+        return node_ref(w, (uint32_t)(m >> (8u * slot)) & 0xffu, (uint32_t)((m << 8) >> (8u * slot)));
+    } else {
+        return node_ref(w, (w[6] >> (8u * slot)) & 0xffu, (w[6] << 8) >> (8u * slot));
     }
 }
 
@@ -102,100 +166,242 @@ __device__ __forceinline__ uint32_t trace_pop(const TraceStack& ts, int& sp, flo
         --sp;
         if (sp >= ts.cap) return EMPTY_CHILD;  // overflowed stack: stop (flagged)
         if (sp < TRACE_LDS) {
-            if (__uint_as_float(ts.lds[(TRACE_LDS + sp) * 64]) > best) continue;
+            // as bits: a best below zero culls nothing
+            if (ts.lds[(TRACE_LDS + sp) * 64] > __float_as_uint(best)) continue;
             return ts.lds[sp * 64];
         }
         return ts.glob[(size_t)(sp - TRACE_LDS) * ts.gstride];
     }
     return EMPTY_CHILD;
 }
-// Closest hit for a ray (origin, direction as stored in the Ray, MinT = tmin,
-// MaxT = FLT_MAX).  Returns false on a miss.  *flags bit 2 is set if the
-// stack capacity was exceeded (the host sizes it from the tree depth, so
-// this never happens for a well-formed build).
+// A closest hit in progress.  Only what cannot be formed again from the ray
+// is kept, so a path kernel can hold it beside the path's state: u, v and the
+// facet come from the hit triangle once the ray is done.
+struct RayTrav {
+    float best;    // distance of the closest hit so far (FLT_MAX: none)
+    int slot;      // its leaf triangle
+    uint32_t ref;  // the node or leaf range to visit next; EMPTY_CHILD: the ray is done
+    int sp;        // stack entries
+    bool tie;
+};
+__device__ __forceinline__ void trav_begin(RayTrav& R) {
+    R.best = 3.40282347e38f;  // FLT_MAX = Ray::m_MaxT
+    R.slot = -1;
+    R.ref = 0;  // root node
+    R.sp = 0;
+    R.tie = false;
+}
+
+// One inner node: the hit children but the nearest are pushed far to near.
+// A child is sorted by its box's entry distance with the slot in the lowest
+// three bits (a distance below the true one, so culling by it stays safe);
+// minima and maxima of one word instead of compared pairs, and its reference
+// is formed only when it is pushed.
 template <int W>
-__device__ bool closest_hit(const SceneDev& S, f3 org, f3 dir, float tmin, const TraceStack& ts, HitRec& h,
-                            uint32_t* flags) {
+__device__ __forceinline__ void trav_node(const SceneDev& S, f3 org, f3 inv, const TraceStack& ts, RayTrav& R,
+                                          uint32_t* flags) {
+    constexpr int NW = node_words(W);
+    uint32_t w[NW];
+    const uint4* nd = reinterpret_cast<const uint4*>(S.nodes + (size_t)R.ref * NW);
+#pragma unroll
+    for (int k = 0; k < NW / 4; ++k) {
+        const uint4 q = nd[k];
+        w[4 * k] = q.x; w[4 * k + 1] = q.y; w[4 * k + 2] = q.z; w[4 * k + 3] = q.w;
+    }
+    const NodeFrame f = node_frame(w, org, inv);
+    uint32_t nx[2], fx[2], ny[2], fy[2], nz[2], fz[2];
+    node_planes<W>(w, 0, inv.x < 0.0f, nx, fx);
+    node_planes<W>(w, 1, inv.y < 0.0f, ny, fy);
+    node_planes<W>(w, 2, inv.z < 0.0f, nz, fz);
+    uint32_t key[W];
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+        const int h = c >> 2, b = c & 3;
+        const float tn = fmaxf(fmaxf(fmaf(byte_f(nx[h], b), f.step.x, f.org.x), fmaf(byte_f(ny[h], b), f.step.y, f.org.y)),
+                               fmaf(byte_f(nz[h], b), f.step.z, f.org.z));
+        const float tf = fminf(fminf(fmaf(byte_f(fx[h], b), f.step.x, f.org.x), fmaf(byte_f(fy[h], b), f.step.y, f.org.y)),
+                               fmaf(byte_f(fz[h], b), f.step.z, f.org.z));
+        // tn <= tf: a ray of NaNs meets nothing
+        const bool hit = (tn <= fminf(tf, R.best)) & (tf >= 0.0f);
+        key[c] = hit ? (__float_as_uint(fmaxf(tn, 0.0f)) & ~7u) | (uint32_t)c : EMPTY_CHILD;
+    }
+    sort_keys<W>(key);
+    if (key[0] == EMPTY_CHILD) {
+        R.ref = trace_pop(ts, R.sp, R.best);
+        return;
+    }
+#pragma unroll
+    for (int c = W - 1; c >= 1; --c) {
+        if (key[c] != EMPTY_CHILD) {
+            const uint32_t r = node_child<W>(w, key[c] & 7u);
+            if (R.sp < TRACE_LDS) {
+                ts.lds[R.sp * 64] = r;
+                ts.lds[(TRACE_LDS + R.sp) * 64] = key[c] & ~7u;
+            }
+            else if (R.sp < ts.cap) ts.glob[(size_t)(R.sp - TRACE_LDS) * ts.gstride] = r;
+            else *flags |= 4u;
+            ++R.sp;
+        }
+    }
+    R.ref = node_child<W>(w, key[0] & 7u);
+}
+
+// A triangle's hit against the closest so far: nearer wins, at the same
+// distance the lower facet.
+__device__ __forceinline__ void trav_take(const SceneDev& S, RayTrav& R, float t, int slot, int fid, bool tied) {
+    if (!(t <= R.best)) return;
+    bool take = t < R.best;
+    if (!take && R.slot >= 0) {
+        const int bf = __float_as_int(S.tri[3 * R.slot].w);
+        R.tie = R.tie || tied || fid != bf;
+        take = fid < bf;
+    } else {
+        R.tie = tied;
+    }
+    if (take) {
+        R.best = t;
+        R.slot = slot;
+    }
+}
+
+// Leaves of the wave: up to 16 of the lanes in `leaves` are served, four of
+// each one's triangles at a time, one triangle per lane.  One lane testing its
+// leaf's triangles in turn would keep the wave for as many dependent loads as
+// the longest leaf has triangles, at six lanes of 64 on average.  own: LDS, the
+// lane served by each group of four.  Called by all active lanes together; act:
+// those lanes.
+template <int Q>
+__device__ __forceinline__ void trav_leaves(const SceneDev& S, f3 org, f3 dir, float tmin, const TraceStack& ts,
+                                            unsigned long long leaves, RayTrav& R) {
+    const int lane = (int)(threadIdx.x & 63u);
+    const int rank = __popcll(leaves & ((1ull << lane) - 1ull));
+    const bool served = ((leaves >> lane) & 1ull) != 0ull && rank < 64 / Q;
+    // lane rank * Q + k tests triangle k of the leaf of the rank-th lane
+    uint32_t* const own = ts.own;
+    if (served) own[rank] = (uint32_t)lane;
+    __builtin_amdgcn_wave_barrier();
+    const int nleaf = min(__popcll(leaves), 64 / Q);
+    const int g = lane / Q, k = lane % Q;
+    const int src = (int)own[min(g, nleaf - 1)];
+    const uint32_t ref = (uint32_t)__shfl((int)R.ref, src, 64);
+    const f3 o = mk(__shfl(org.x, src, 64), __shfl(org.y, src, 64), __shfl(org.z, src, 64));
+    const f3 d = mk(__shfl(dir.x, src, 64), __shfl(dir.y, src, 64), __shfl(dir.z, src, 64));
+    const int cnt = (int)(ref & 7u) + 1;
+    int s = (int)((ref & ~LEAF_BIT) >> 3) + min(k, cnt - 1);
+    float t, u, v;
+    int fid;
+    if (!(tri_test(S.tri, s, o, d, t, u, v, fid) && t > tmin)) t = __int_as_float(0x7f800000);
+    bool tied = false;
+#pragma unroll
+    for (int off = 1; off < Q; off <<= 1) {
+        const float t2 = __shfl_xor(t, off, 64);
+        const int f2 = __shfl_xor(fid, off, 64), s2 = __shfl_xor(s, off, 64);
+        const bool ti2 = __shfl_xor((int)tied, off, 64) != 0;
+        const bool eq = t2 == t, sw = t2 < t || (eq && f2 < fid);
+        tied = eq ? (tied || ti2 || f2 != fid) : (sw ? ti2 : tied);
+        t = sw ? t2 : t;
+        fid = sw ? f2 : fid;
+        s = sw ? s2 : s;
+    }
+    // back to the ray's lane
+    const int from = (rank * Q) & 63;
+    const float rt = __shfl(t, from, 64);
+    const int rf = __shfl(fid, from, 64), rs = __shfl(s, from, 64), ri = __shfl((int)tied, from, 64);
+    if (served) {
+        if (rt < __int_as_float(0x7f800000)) trav_take(S, R, rt, rs, rf, ri != 0);
+        // the leaf's other triangles, if any
+        R.ref = (R.ref & 7u) >= (uint32_t)Q ? R.ref + 8u * Q - Q : trace_pop(ts, R.sp, R.best);
+    }
+}
+
+// The triangles of a lane's own leaf.
+__device__ __forceinline__ void trav_leaf(const SceneDev& S, f3 org, f3 dir, float tmin, const TraceStack& ts,
+                                          RayTrav& R) {
+    const int s0 = (int)((R.ref & ~LEAF_BIT) >> 3), s1 = s0 + (int)(R.ref & 7u);
+    for (int s = s0; s <= s1; ++s) {
+        float t, u, v;
+        int fid;
+        if (tri_test(S.tri, s, org, dir, t, u, v, fid) && t > tmin) trav_take(S, R, t, s, fid, false);
+    }
+    R.ref = trace_pop(ts, R.sp, R.best);
+}
+
+// Runs the wave's rays (lanes whose ref is not EMPTY_CHILD) until at most
+// `stop` of them are left.  A step is either an inner node for the lanes that
+// stand at one or leaves for the others, whichever more lanes ask for (a leaf
+// step costs about two thirds of a node's, so half as many lanes are enough for
+// it), so a lane at a leaf does not sit through another lane's node or the
+// other way round.
+// WAVE: the whole wave calls this together, and its lanes share the leaves'
+// triangles; eight lanes for a leaf (all its triangles) where no more than
+// eight lanes stand at one, else four.  Otherwise the lanes that call it are
+// the wave, and each tests its own leaf.
+constexpr int TRAV_LEAF_VOTE = 2;
+template <int W, bool WAVE>
+__device__ __forceinline__ void trav_run(const SceneDev& S, f3 org, f3 dir, float tmin, const TraceStack& ts, int stop,
+                                         RayTrav& R, uint32_t* flags) {
     const float BIG = 1e16f;
     f3 inv;
     inv.x = fabs_(dir.x) < 1e-16f ? (dir.x > 0.0f ? BIG : -BIG) : 1.0f / dir.x;
     inv.y = fabs_(dir.y) < 1e-16f ? (dir.y > 0.0f ? BIG : -BIG) : 1.0f / dir.y;
     inv.z = fabs_(dir.z) < 1e-16f ? (dir.z > 0.0f ? BIG : -BIG) : 1.0f / dir.z;
-    const f3 oi = mk(org.x * inv.x, org.y * inv.y, org.z * inv.z);
-    float best = 3.40282347e38f;  // FLT_MAX = Ray::m_MaxT
-    int bfacet = 0x7fffffff;
-    int bslot = -1;
-    float bu = 0.0f, bv = 0.0f;
-    bool tie = false;
-    const int NF = node_floats(W);
-    int sp = 0;
-    uint32_t ref = 0;  // root node
     for (;;) {
-        if (ref & LEAF_BIT) {
-            int start = (int)((ref & ~LEAF_BIT) >> 3);
-            int count = (int)(ref & 7u) + 1;
-            for (int k = 0; k < count; ++k) {
-                int s = start + k;
-                float t, u, v;
-                if (tri_test(S.tri, s, org, dir, t, u, v)) {
-                    int fid = __float_as_int(S.tri[3 * s].w);
-                    if (t > tmin) {
-                        tie = t == best ? (tie || fid != bfacet) : (t < best ? false : tie);
-                        if (t < best || (t == best && fid < bfacet)) {
-                            best = t; bu = u; bv = v; bfacet = fid; bslot = s;
-                        }
-                    }
-                }
+        const bool on = R.ref != EMPTY_CHILD;
+        const bool leaf = on && (R.ref & LEAF_BIT) != 0u;
+        const unsigned long long leaves = __ballot(leaf);
+        const int nl = __popcll(leaves), nn = __popcll(__ballot(on && !leaf));
+        if (nl + nn <= stop) break;
+        if (nl * TRAV_LEAF_VOTE >= nn) {
+            if constexpr (WAVE) {
+                if (nl <= 8) trav_leaves<8>(S, org, dir, tmin, ts, leaves, R);
+                else trav_leaves<4>(S, org, dir, tmin, ts, leaves, R);
+            } else if (leaf) {
+                trav_leaf(S, org, dir, tmin, ts, R);
             }
         } else {
-            const float* nd = S.nodes + (size_t)ref * NF;
-            float d[W];
-            uint32_t r[W];
-            const uint32_t* cref = reinterpret_cast<const uint32_t*>(nd + 6 * W);
-#pragma unroll
-            for (int c = 0; c < W; ++c) {
-                float tx0 = fmaf(nd[0 * W + c], inv.x, -oi.x), tx1 = fmaf(nd[3 * W + c], inv.x, -oi.x);
-                float ty0 = fmaf(nd[1 * W + c], inv.y, -oi.y), ty1 = fmaf(nd[4 * W + c], inv.y, -oi.y);
-                float tz0 = fmaf(nd[2 * W + c], inv.z, -oi.z), tz1 = fmaf(nd[5 * W + c], inv.z, -oi.z);
-                float tn = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fminf(tz0, tz1));
-                float tf = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fmaxf(tz0, tz1));
-                uint32_t cr = cref[c];
-                bool hit = (cr != EMPTY_CHILD) && (tf >= tn) && (tn <= best) && (tf >= 0.0f);
-                d[c] = hit ? tn : 3.0e38f;
-                r[c] = hit ? cr : EMPTY_CHILD;
-            }
-            sort_children<W>(d, r);
-            if (r[0] != EMPTY_CHILD) {
-                // push the farther children far-to-near, descend into the nearest
-#pragma unroll
-                for (int c = W - 1; c >= 1; --c) {
-                    if (r[c] != EMPTY_CHILD) {
-                        if (sp < TRACE_LDS) {
-                            ts.lds[sp * 64] = r[c];
-                            ts.lds[(TRACE_LDS + sp) * 64] = __float_as_uint(d[c]);
-                        }
-                        else if (sp < ts.cap) ts.glob[(size_t)(sp - TRACE_LDS) * ts.gstride] = r[c];
-                        else *flags |= 4u;
-                        ++sp;
-                    }
-                }
-                ref = r[0];
-                continue;
-            }
+            if (on && !leaf) trav_node<W>(S, org, inv, ts, R, flags);
         }
-        ref = trace_pop(ts, sp, best);
-        if (ref == EMPTY_CHILD) break;
     }
-    if (bslot < 0 || !(best < 3.40282347e38f)) {
+}
+
+// The hit of a ray that is done; false: a miss.
+__device__ __forceinline__ bool trav_hit(const SceneDev& S, f3 org, f3 dir, const RayTrav& R, HitRec& h) {
+    if (R.slot < 0 || !(R.best < 3.40282347e38f)) {
         h.facet = -1;
         h.slot = -1;
         h.t = 3.40282347e38f;
         h.tie = false;
         return false;
     }
-    h.t = best; h.u = bu; h.v = bv; h.facet = bfacet; h.slot = bslot;
-    h.tie = tie;
+    float t;
+    tri_test(S.tri, R.slot, org, dir, t, h.u, h.v, h.facet);
+    h.t = R.best;
+    h.slot = R.slot;
+    h.tie = R.tie;
     return true;
+}
+
+// Closest hit for a ray (origin, direction as stored in the Ray, MinT = tmin,
+// MaxT = FLT_MAX).  Returns false on a miss.  *flags bit 2 is set if the
+// stack capacity was exceeded (the host sizes it from the tree depth, so
+// this never happens for a well-formed build).
+template <int W>
+__device__ __forceinline__ bool closest_hit(const SceneDev& S, f3 org, f3 dir, float tmin, const TraceStack& ts,
+                                            HitRec& h, uint32_t* flags) {
+    RayTrav R;
+    trav_begin(R);
+    trav_run<W, false>(S, org, dir, tmin, ts, 0, R, flags);
+    return trav_hit(S, org, dir, R, h);
+}
+// The same for a whole wave; on: the lane has a ray.
+template <int W>
+__device__ __forceinline__ bool closest_hit_wave(const SceneDev& S, bool on, f3 org, f3 dir, float tmin,
+                                                 const TraceStack& ts, HitRec& h, uint32_t* flags) {
+    RayTrav R;
+    trav_begin(R);
+    if (!on) R.ref = EMPTY_CHILD;
+    trav_run<W, true>(S, org, dir, tmin, ts, 0, R, flags);
+    return on && trav_hit(S, org, dir, R, h);
 }
 
 // ---- calculateGeometry (SPPM.cpp:36-77) ------------------------------------

@@ -48,8 +48,6 @@ constexpr int HIT_TIE = 0x40000000;        // hit record: tie flag beside the le
 constexpr float F_MAX = 3.40282347e38f;    // Ray::m_MaxT
 
 // ---- path state ----------------------------------------------------------
-// MT cursor: ia = 1 + k and ib = 397 + k hold for every cursor (mt_seed
-// starts at k = 0, ia = 1, ib = 397 and mt_next advances all three).
 __device__ __forceinline__ void path_store(const PathStateDev& Q, const PhotonPath& P) {
     const int i = P.i;
     Q.rng[i] = make_uint4(P.m.a0, P.m.a1, P.m.b, P.m.k);
@@ -64,7 +62,6 @@ __device__ __forceinline__ void path_load(const PathStateDev& Q, int i, PhotonPa
     P.i = i;
     const uint4 m = Q.rng[i];
     P.m.a0 = m.x; P.m.a1 = m.y; P.m.b = m.z; P.m.k = m.w;
-    P.m.ia = 1u + m.w; P.m.ib = 397u + m.w;
     const float4 o = Q.org[i], d = Q.dir[i], n = Q.ndir[i], r = Q.rad[i], t = Q.thr[i];
     P.cur_org = mk(o.x, o.y, o.z); P.cur_index = o.w;
     P.cur_dir = mk(d.x, d.y, d.z); P.next_index = d.w;
@@ -101,8 +98,9 @@ __global__ void __launch_bounds__(256) k_pw_emit(SceneDev S, SlotsDev slots, int
     if (i >= N) return;
     uint32_t ovf = 0;
     PhotonPath P;
-    if constexpr (GUIDED) photon_start_guided(S, slots, G, N, step, i, P, &ovf);
-    else photon_start(S, slots, N, step, i, P, &ovf);
+    const uint32_t w397 = mt_word397(photon_seed(N, step, i));
+    if constexpr (GUIDED) photon_start_guided(S, slots, G, N, step, i, w397, P, &ovf);
+    else photon_start(S, slots, N, step, i, w397, P, &ovf);
     photon_pretrace(P);
     path_store(Q, P);
     ray_store(rays, i, P);
@@ -132,7 +130,7 @@ __global__ void __launch_bounds__(WT_BLOCK, WT_MIN_WAVES) k_pw_trace(
     unsigned long long* __restrict__ counts) {
     constexpr int G = 64 / L;     // rays per wave
     constexpr int CPL = W / L;    // children per lane at an inner node
-    constexpr int NF = node_floats(W);
+    constexpr int NF = node_words(W);
     __shared__ uint32_t stk[WT_WAVES * G][WT_LDS + 1];  // +1: a group's entries start in another bank
     const int lane = threadIdx.x & 63;
     const int c = lane & (L - 1);
@@ -152,7 +150,7 @@ __global__ void __launch_bounds__(WT_BLOCK, WT_MIN_WAVES) k_pw_trace(
     int pbase = 0, pend = 0;  // the wave's pool of queue entries [pbase, pend)
     int q = 0, sp = 0;
     uint32_t ref = 0;
-    f3 org = mk(0.0f, 0.0f, 0.0f), dir = org, inv = org, oi = org;
+    f3 org = mk(0.0f, 0.0f, 0.0f), dir = org, inv = org;
     float best = F_MAX, bu = 0.0f, bv = 0.0f;
     int bfacet = 0x7fffffff, bslot = -1;
     bool tie = false;
@@ -179,7 +177,6 @@ __global__ void __launch_bounds__(WT_BLOCK, WT_MIN_WAVES) k_pw_trace(
                     inv.x = fabs_(dir.x) < 1e-16f ? (dir.x > 0.0f ? BIG : -BIG) : 1.0f / dir.x;
                     inv.y = fabs_(dir.y) < 1e-16f ? (dir.y > 0.0f ? BIG : -BIG) : 1.0f / dir.y;
                     inv.z = fabs_(dir.z) < 1e-16f ? (dir.z > 0.0f ? BIG : -BIG) : 1.0f / dir.z;
-                    oi = mk(org.x * inv.x, org.y * inv.y, org.z * inv.z);
                     best = F_MAX; bu = 0.0f; bv = 0.0f; bfacet = 0x7fffffff; bslot = -1; tie = false;
                     sp = 0;
                     ref = 0;  // root
@@ -212,8 +209,8 @@ __global__ void __launch_bounds__(WT_BLOCK, WT_MIN_WAVES) k_pw_trace(
                 for (int k = c; k < count; k += L) {
                     const int s = start + k;
                     float t, u, v;
-                    if (tri_test(S.tri, s, org, dir, t, u, v)) {
-                        const int fid = __float_as_int(S.tri[3 * s].w);
+                    int fid;
+                    if (tri_test(S.tri, s, org, dir, t, u, v, fid)) {
                         if (t > tmin) {
                             ltie = t == lt ? (ltie || fid != lf) : (t < lt ? false : ltie);
                             if (t < lt || (t == lt && fid < lf)) {
@@ -253,7 +250,10 @@ __global__ void __launch_bounds__(WT_BLOCK, WT_MIN_WAVES) k_pw_trace(
                 }
                 pop = true;
             } else {
-                const float* nd = S.nodes + (size_t)ref * NF + c * CPL;
+                const uint32_t* nd = S.nodes + (size_t)ref * NF;
+                const unsigned char* meta = reinterpret_cast<const unsigned char*>(nd + 6) + c * CPL;
+                const unsigned char* planes = reinterpret_cast<const unsigned char*>(nd + NODE_PLANES(W)) + c * CPL;
+                const NodeFrame f = node_frame(nd, org, inv);
                 float d[CPL];
                 uint32_t cr[CPL];
                 bool hit[CPL];
@@ -261,15 +261,17 @@ __global__ void __launch_bounds__(WT_BLOCK, WT_MIN_WAVES) k_pw_trace(
                 int nh = 0;
 #pragma unroll
                 for (int k = 0; k < CPL; ++k) {
-                    const float bx0 = nd[0 * W + k], by0 = nd[1 * W + k], bz0 = nd[2 * W + k];
-                    const float bx1 = nd[3 * W + k], by1 = nd[4 * W + k], bz1 = nd[5 * W + k];
-                    cr[k] = __float_as_uint(nd[6 * W + k]);
-                    const float tx0 = fmaf(bx0, inv.x, -oi.x), tx1 = fmaf(bx1, inv.x, -oi.x);
-                    const float ty0 = fmaf(by0, inv.y, -oi.y), ty1 = fmaf(by1, inv.y, -oi.y);
-                    const float tz0 = fmaf(bz0, inv.z, -oi.z), tz1 = fmaf(bz1, inv.z, -oi.z);
+                    cr[k] = node_ref(nd, meta[k], c * CPL + k > 0 ? meta[k - 1] : 0u);
+                    const float tx0 = fmaf((float)planes[0 * W + k], f.step.x, f.org.x);
+                    const float tx1 = fmaf((float)planes[1 * W + k], f.step.x, f.org.x);
+                    const float ty0 = fmaf((float)planes[2 * W + k], f.step.y, f.org.y);
+                    const float ty1 = fmaf((float)planes[3 * W + k], f.step.y, f.org.y);
+                    const float tz0 = fmaf((float)planes[4 * W + k], f.step.z, f.org.z);
+                    const float tz1 = fmaf((float)planes[5 * W + k], f.step.z, f.org.z);
+                    const bool used = planes[0 * W + k] <= planes[1 * W + k];
                     const float tn = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fminf(tz0, tz1));
                     const float tf = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fmaxf(tz0, tz1));
-                    hit[k] = (cr[k] != EMPTY_CHILD) && (tf >= tn) && (tn <= best) && (tf >= 0.0f);
+                    hit[k] = used && (tf >= tn) && (tn <= best) && (tf >= 0.0f);
                     d[k] = hit[k] ? tn : 3.0e38f;
                     hm[k] = __ballot(hit[k]) & gmask;
                     nh += __popcll(hm[k]);
@@ -402,7 +404,7 @@ __global__ void __launch_bounds__(PATH_BLOCK, PATH_WAVES_PER_SIMD) k_pw_resume(
     unsigned long long* __restrict__ counts) {
     __shared__ uint32_t stk[TRACE_STACK_WORDS];
     const int lane = threadIdx.x;
-    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap};
+    const TraceStack ts{stk + lane, spill + (size_t)blockIdx.x * PATH_BLOCK + lane, (int)gridDim.x * PATH_BLOCK, cap, stk + 2 * TRACE_LDS * 64};
     const unsigned long long below = (1ull << lane) - 1ull;
     uint32_t ovf = 0, fl = 0, nray = 0, ntie = 0;
     PhotonPath P;

@@ -53,6 +53,32 @@ def test_closest_hit_bit_exact(width, which, builder, box_scene, full_scene_smal
     np.testing.assert_array_equal(vg[hit], vo[hit])
 
 
+@pytest.mark.parametrize("width", [2, 4, 8])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1024, 1025, 2049, 65537])
+def test_ray_counts_split_over_waves(n, width):
+    """Closest hits and occlusion for ray counts around the sizes where the
+    rays per wave change (1024 waves take one ray each first, 64 at most):
+    against brute force, ties and triangle counts per leaf of all sizes."""
+    scene = scenes.screens_scene()
+    say(f"ray counts: n={n} width={width}")
+    org, d = random_rays(scene, max(n, 16), seed=n + width)
+    org, d = org[-n:], d[-n:]
+    os_ = pyoracle.OracleScene(scene)
+    r = sppm_amd.Renderer(scene, scenes.pinhole_camera(8, 8), 0.9, 0.015, 64, bvh_width=width)
+    for got, want in zip(r.trace(org, d), os_.closest_hit(org, d, mode=0)):
+        np.testing.assert_array_equal(got, want)
+    tmax = np.random.default_rng(n).uniform(0.02, 1.8, size=n).astype(np.float32)
+    np.testing.assert_array_equal(r.occluded(org, d, 1e-4, tmax, 0.5), os_.occluded(org, d, 1e-4, tmax, 0.5))
+    r.close()
+
+
+@pytest.mark.parametrize("w,h,N", [(1, 1, 1), (3, 1, 63), (32, 32, 1025), (33, 31, 17000)])
+def test_pass_parity_path_counts_split_over_waves(w, h, N, full_scene_small):
+    """Whole passes at path and pixel counts around the sizes where the share
+    of a wave changes, on the scene with every material."""
+    run_parity(full_scene_small, scenes.thinlens_camera(w, h), 0.9, 0.05, N, 2, 8, f"path counts {w}x{h} {N}")
+
+
 def small_scene(case):
     """The light quad plus a few triangles: random ones (2, 3, 5, 9, 33 in
     all), 64 coincident copies of one triangle (every centroid extent zero:
