@@ -36,9 +36,9 @@ namespace sppm {
 // pixel order, 6 words per pixel.  The block of a pass (6 * pixels words) is
 // cut into K segments of L words; segment k's state window (where it
 // starts) comes from the host for the first pass.
-//   k_camw_emit  one wave per segment emits the segment's tempered words and
+//   k_camw_emit  one workgroup per segment emits the segment's tempered words and
 //                stores the window after it;
-//   k_camw_jump  one workgroup per segment jumps that window over the other
+//   k_camw_jump  CAMW_JUMP_PARTS workgroups per segment jump that window over the other
 //                K - 1 segments (t^((K-1)L) mod P applied as a sum of shifted
 //                windows): the start of its segment in the next pass.
 // Raw word x[m], m >= 624, is mix(x[m-624], x[m-623], x[m-227]), so 227
@@ -58,41 +58,47 @@ __device__ __forceinline__ uint32_t mt_mix(uint32_t a, uint32_t b, uint32_t c) {
 }
 constexpr int CAMW_RING = 1024;       // raw words kept (>= 624 + 227, and >= 227 + 624 for the jump's reads)
 constexpr int CAMW_DEG = 19937;       // degree of the characteristic polynomial
+constexpr int CAMW_EMIT_THREADS = 256;  // 227 words a step
 constexpr int CAMW_JUMP_THREADS = 640;  // 624 output words of the jumped window
+constexpr int CAMW_JUMP_PARTS = 8;      // workgroups that share a segment's jump
 
-// One wave per segment: x[624 + q] -> out[q] for q < L, 227 words per step
-// in four rounds of 64 lanes.  A step reads only words of earlier steps, and
-// the wave's LDS accesses are executed in order, so no barrier is needed.
+// One workgroup per segment: x[624 + q] -> out[q] for q < L, 227 words per
+// step, a word per thread.  A step reads only words of earlier steps, so one
+// barrier a step is enough (what it overwrites was last read 1024 words ago).
+// A serial chain of LDS round trips bounds it: one wave with four words per
+// lane took 460 ns a step, four waves 150.  The segment's window is
+// cleared once it is read: the jump adds the next one up there.
 // segment seg of a stream: states, words and ends as for launch_camera_words
-__device__ __forceinline__ void camw_emit(const uint32_t* __restrict__ states, long long L,
+__device__ __forceinline__ void camw_emit(uint32_t* __restrict__ states, long long L,
                                           uint32_t* __restrict__ words, uint32_t* __restrict__ ends, int seg,
                                           uint32_t* ring) {
-    const int lane = threadIdx.x;
-    const uint32_t* st = states + (size_t)seg * 624;
-    for (int k = lane; k < 624; k += 64) ring[k] = st[k];
-    __builtin_amdgcn_wave_barrier();
+    const int t = threadIdx.x;
+    uint32_t* st = states + (size_t)seg * 624;
+    for (int k = t; k < 624; k += CAMW_EMIT_THREADS) {
+        ring[k] = st[k];
+        st[k] = 0u;
+    }
+    __syncthreads();
     uint32_t* out = words + (size_t)seg * (size_t)L;
     const long long mend = 624 + L;
     for (long long m0 = 624; m0 < mend; m0 += 227) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int idx = r * 64 + lane;
-            const long long m = m0 + idx;
-            if (idx < 227 && m < mend) {
-                const uint32_t x = mt_mix(ring[(m - 624) & (CAMW_RING - 1)], ring[(m - 623) & (CAMW_RING - 1)],
-                                          ring[(m - 227) & (CAMW_RING - 1)]);
-                ring[m & (CAMW_RING - 1)] = x;
-                out[m - 624] = temper(x);
-            }
+        const long long m = m0 + t;
+        if (t < 227 && m < mend) {
+            const int r = (int)(m & (CAMW_RING - 1));
+            const uint32_t x = mt_mix(ring[(r - 624) & (CAMW_RING - 1)], ring[(r - 623) & (CAMW_RING - 1)],
+                                      ring[(r - 227) & (CAMW_RING - 1)]);
+            ring[r] = x;
+            out[m - 624] = temper(x);
         }
-        __builtin_amdgcn_wave_barrier();
+        __syncthreads();
     }
     // the window after the segment: x[L .. L + 623]
     uint32_t* e = ends + (size_t)seg * 624;
-    for (int j = lane; j < 624; j += 64) e[j] = ring[(L + j) & (CAMW_RING - 1)];
+    for (int j = t; j < 624; j += CAMW_EMIT_THREADS) e[j] = ring[(L + j) & (CAMW_RING - 1)];
 }
-__global__ void __launch_bounds__(64) k_camw_emit(const uint32_t* __restrict__ states, long long L,
-                                                  uint32_t* __restrict__ words, uint32_t* __restrict__ ends) {
+__global__ void __launch_bounds__(CAMW_EMIT_THREADS) k_camw_emit(uint32_t* __restrict__ states, long long L,
+                                                                 uint32_t* __restrict__ words,
+                                                                 uint32_t* __restrict__ ends) {
     __shared__ uint32_t ring[CAMW_RING];
     camw_emit(states, L, words, ends, (int)blockIdx.x, ring);
 }
@@ -101,47 +107,62 @@ __global__ void __launch_bounds__(64) k_camw_emit(const uint32_t* __restrict__ s
 // y[k] = x[L + k].  The coefficients are taken 227 at a time; before a block
 // [i0, i0 + 227) the words up to y[i0 + 226 + 623] are generated into the
 // ring (227 at a time, one barrier), whose oldest slot then holds y[i0 - 175]
-// or later, so the block's reads y[i0 ..] are intact.
+// or later, so the block's reads y[i0 ..] are intact.  Its first 32 words
+// are kept once more behind its end, so that 32 coefficients read at fixed
+// offsets from one address.  Part `part` of CAMW_JUMP_PARTS takes its share of
+// the blocks (it generates the words before them too, 88 steps at most) and
+// adds its sum into the cleared window.  One workgroup for the whole jump,
+// one dependent LDS read per set coefficient: 0.52 ms, which the camera words
+// of renders below 512^2 pixels waited for.
 __device__ __forceinline__ void camw_jump(const uint32_t* __restrict__ ends, const uint32_t* __restrict__ phi,
-                                          uint32_t* __restrict__ states, int seg, uint32_t* ring) {
+                                          uint32_t* __restrict__ states, int seg, int part, uint32_t* ring) {
     const int t = threadIdx.x;
     const uint32_t* e = ends + (size_t)seg * 624;
-    if (t < 624) ring[t] = e[t];  // y[k] at ring[k & 1023]
+    if (t < 624) {
+        ring[t] = e[t];  // y[k] at ring[k & 1023]
+        if (t < 32) ring[CAMW_RING + t] = e[t];
+    }
     __syncthreads();
+    constexpr int NBLK = (CAMW_DEG + 226) / 227;
+    constexpr int PER = (NBLK + CAMW_JUMP_PARTS - 1) / CAMW_JUMP_PARTS;
+    const int b1 = min((part + 1) * PER, NBLK);
     uint32_t acc = 0;
     int gen = 623;  // highest y generated
-    for (int i0 = 0; i0 < CAMW_DEG; i0 += 227) {
+    for (int blk = 0; blk < b1; ++blk) {
+        const int i0 = blk * 227;
         const int i1 = i0 + 227 < CAMW_DEG ? i0 + 227 : CAMW_DEG;
         const int need = i1 - 1 + 623;
         if (t < need - gen) {
-            const int k = gen + 1 + t;
-            ring[k & (CAMW_RING - 1)] = mt_mix(ring[(k - 624) & (CAMW_RING - 1)], ring[(k - 623) & (CAMW_RING - 1)],
-                                               ring[(k - 227) & (CAMW_RING - 1)]);
+            const int k = gen + 1 + t, r = k & (CAMW_RING - 1);
+            const uint32_t x = mt_mix(ring[(k - 624) & (CAMW_RING - 1)], ring[(k - 623) & (CAMW_RING - 1)],
+                                      ring[(k - 227) & (CAMW_RING - 1)]);
+            ring[r] = x;
+            if (r < 32) ring[CAMW_RING + r] = x;
         }
         gen = need;
         __syncthreads();
-        if (t < 624) {
-            for (int w = i0 >> 5; w <= (i1 - 1) >> 5; ++w) {
-                uint32_t bits = phi[w];
-                const int lo = i0 - w * 32, hi = i1 - w * 32;
-                if (lo > 0) bits &= ~((1u << lo) - 1u);
-                if (hi < 32) bits &= (1u << hi) - 1u;
-                while (bits) {
-                    const int b = __builtin_ctz(bits);
-                    bits &= bits - 1u;
-                    acc ^= ring[(w * 32 + b + t) & (CAMW_RING - 1)];
+        if (blk >= part * PER) {
+            if (t < 624) {
+                for (int w = i0 >> 5; w <= (i1 - 1) >> 5; ++w) {
+                    uint32_t bits = phi[w];
+                    const int lo = i0 - w * 32, hi = i1 - w * 32;
+                    if (lo > 0) bits &= ~((1u << lo) - 1u);
+                    if (hi < 32) bits &= (1u << hi) - 1u;
+                    const uint32_t* y = ring + ((w * 32 + t) & (CAMW_RING - 1));
+#pragma unroll
+                    for (int b = 0; b < 32; ++b) acc ^= y[b] & (uint32_t)((int)(bits << (31 - b)) >> 31);
                 }
             }
+            __syncthreads();
         }
-        __syncthreads();
     }
-    if (t < 624) states[(size_t)seg * 624 + t] = acc;
+    if (t < 624) atomicXor(&states[(size_t)seg * 624 + t], acc);
 }
 __global__ void __launch_bounds__(CAMW_JUMP_THREADS) k_camw_jump(const uint32_t* __restrict__ ends,
                                                                  const uint32_t* __restrict__ phi,
                                                                  uint32_t* __restrict__ states) {
-    __shared__ uint32_t ring[CAMW_RING];
-    camw_jump(ends, phi, states, (int)blockIdx.x, ring);
+    __shared__ uint32_t ring[CAMW_RING + 32];
+    camw_jump(ends, phi, states, (int)blockIdx.x / CAMW_JUMP_PARTS, (int)blockIdx.x % CAMW_JUMP_PARTS, ring);
 }
 
 // The camera words of every scene of a batch: block b is segment b -
@@ -154,7 +175,7 @@ __device__ __forceinline__ int owner_of(const int* __restrict__ start, int n, in
     }
     return lo;
 }
-__global__ void __launch_bounds__(64) k_camw_emit_multi(const CamJob* __restrict__ jobs,
+__global__ void __launch_bounds__(CAMW_EMIT_THREADS) k_camw_emit_multi(const CamJob* __restrict__ jobs,
                                                         const int* __restrict__ kstart, int njobs) {
     __shared__ uint32_t ring[CAMW_RING];
     const int s = owner_of(kstart, njobs, (int)blockIdx.x);
@@ -163,10 +184,11 @@ __global__ void __launch_bounds__(64) k_camw_emit_multi(const CamJob* __restrict
 }
 __global__ void __launch_bounds__(CAMW_JUMP_THREADS) k_camw_jump_multi(const CamJob* __restrict__ jobs,
                                                                        const int* __restrict__ kstart, int njobs) {
-    __shared__ uint32_t ring[CAMW_RING];
-    const int s = owner_of(kstart, njobs, (int)blockIdx.x);
+    __shared__ uint32_t ring[CAMW_RING + 32];
+    const int b = (int)blockIdx.x / CAMW_JUMP_PARTS;
+    const int s = owner_of(kstart, njobs, b);
     const CamJob& J = jobs[s];
-    camw_jump(J.states + (size_t)J.K * 624, J.phi, J.states, (int)blockIdx.x - kstart[s], ring);
+    camw_jump(J.states + (size_t)J.K * 624, J.phi, J.states, b - kstart[s], (int)blockIdx.x % CAMW_JUMP_PARTS, ring);
 }
 
 // Persistent photon pass.  A wave claims path indices from the striped path
@@ -1709,12 +1731,12 @@ int trace_grid_blocks(int width) {
 
 void launch_camera_words(uint32_t* states, const uint32_t* phi, int K, long long L, uint32_t* words, hipStream_t st) {
     uint32_t* ends = states + (size_t)K * 624;  // scratch: the windows after the segments
-    hipLaunchKernelGGL(k_camw_emit, dim3(K), dim3(64), 0, st, states, L, words, ends);
-    hipLaunchKernelGGL(k_camw_jump, dim3(K), dim3(CAMW_JUMP_THREADS), 0, st, ends, phi, states);
+    hipLaunchKernelGGL(k_camw_emit, dim3(K), dim3(CAMW_EMIT_THREADS), 0, st, states, L, words, ends);
+    hipLaunchKernelGGL(k_camw_jump, dim3(K * CAMW_JUMP_PARTS), dim3(CAMW_JUMP_THREADS), 0, st, ends, phi, states);
 }
 void launch_camera_words_multi(const CamJob* jobs, const int* kstart, int njobs, int nseg, hipStream_t st) {
-    hipLaunchKernelGGL(k_camw_emit_multi, dim3(nseg), dim3(64), 0, st, jobs, kstart, njobs);
-    hipLaunchKernelGGL(k_camw_jump_multi, dim3(nseg), dim3(CAMW_JUMP_THREADS), 0, st, jobs, kstart, njobs);
+    hipLaunchKernelGGL(k_camw_emit_multi, dim3(nseg), dim3(CAMW_EMIT_THREADS), 0, st, jobs, kstart, njobs);
+    hipLaunchKernelGGL(k_camw_jump_multi, dim3(nseg * CAMW_JUMP_PARTS), dim3(CAMW_JUMP_THREADS), 0, st, jobs, kstart, njobs);
 }
 
 // Items (paths, pixels, rays) a wave takes at a time: as many as there are for

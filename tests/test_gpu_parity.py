@@ -214,6 +214,14 @@ def test_pass_parity_gather_edges(box_scene, w, h, N, r0):
                record=sppm_amd.RECORD_PAIRS, max_pairs=40_000_000)
 
 
+@pytest.mark.parametrize("w,h", [(1, 1), (2, 1), (37, 1), (38, 1), (227, 1), (119, 61)])
+def test_camera_words_sizes(w, h, box_scene):
+    """Three passes' camera words at sizes around the generator's own (227 words
+    a step, 624 a window, segments of one word to thousands), through the hit
+    points, against the oracle's sequential stream."""
+    run_parity(box_scene, scenes.pinhole_camera(w, h), 0.9, 0.05, 500, 3, 4, f"camera words {w}x{h}")
+
+
 def test_pass_parity_environment_light():
     """Box lit also by an environment map through its open side: eye paths
     continue past their hit points and add the sky when they leave
