@@ -107,6 +107,10 @@ struct SceneBuffers {
 
 struct RenderBuffers {
     bool ready = false;
+    // what the buffers were allocated for: another sppm_begin of the same
+    // sizes fills them anew instead of freeing and allocating them (2 to 10 ms
+    // of a render's time)
+    std::vector<long long> shape;
     int N = 0, W = 0, H = 0, np = 0;
     SlotsDev slots{};
     int* off = nullptr;
@@ -189,6 +193,8 @@ struct RenderBuffers {
         hits = HitDev{};
         dfree(shared.rad); dfree(shared.cnt); dfree(shared.direct); dfree(counts); dfree(list_off); dfree(list_scan_tmp); dfree(lists);
         dfree(words); dfree(cam_states); dfree(cam_phi); dfree(rstat); dfree(tiles); dfree(chunkp); dfree(nch); dfree(chunk_off); dfree(tile_scan_tmp); dfree(partial); dfree(groups.keys); dfree(groups.vals); dfree(groups.tmp_k); dfree(groups.tmp_v); dfree(groups.hist); dfree(groups.nvalid); dfree(groups.chunkq); dfree(groups.stat); dfree(groups.spheres); dfree(pass_dev); dfree(path_cell); dfree(path_ratio); dfree(pdep); dfree(doff); dfree(flags); dfree(ctr); dfree(raystripes); dfree(image);
+        lists_cap = 0;
+        shape.clear();
         ready = false;
     }
 };
@@ -960,8 +966,9 @@ static int init_camera_stream(sppm_ctx* c) {
             break;
         }
     const long long L = block / K;
-    int rc = dalloc(&R.cam_states, 2 * (size_t)K * MT_WORDS);  // the windows, then scratch for the kernels
-    if (rc) return rc;
+    // the windows, then scratch for the kernels
+    if (!R.cam_states)
+        if (int rc = dalloc(&R.cam_states, 2 * (size_t)K * MT_WORDS)) return rc;
     std::vector<uint32_t> win((size_t)K * MT_WORDS);
     mt_window_seed((uint32_t)c->cam.sampler_id, win.data());
     for (int k = 1; k < K; ++k) {
@@ -997,101 +1004,112 @@ int sppm_begin(sppm_ctx* c) {
     c->eye_recorded[0] = c->eye_recorded[1] = false;
     drop_graph(c);
     RenderBuffers& R = c->rb;
-    R.release();
+    R.ready = false;
     const int N = c->params.photons_per_pass;
     const int W = c->cam.width, Hh = c->cam.height, np = W * Hh;
-    R.N = N; R.W = W; R.H = Hh; R.np = np;
     R.photon_cap = N * (NSLOT - 1);  // checked against RADIX_SORT_MAX_N by sppm_params_set
     R.cell_cap = 1 << 22;
     const size_t NS = (size_t)NSLOT * N;
     int rc = 0;
-    // tiles of the recording gather (8x8 pixels) or hit-point groups of the production gather
-    const int ntile_max = std::max(gather_tile_count(W, Hh), gather_group_count(np));
-    R.slots.npaths = N;
-    if ((rc = dalloc(&R.slots.pos, NS)) || (rc = dalloc(&R.slots.flux, NS)) || (rc = dalloc(&R.slots.dir, NS)) ||
-        (rc = dalloc(&R.slots.valid, NS)) || (rc = dalloc(&R.slots.count, N)) || (rc = dalloc(&R.off, N)) ||
-        (rc = dalloc(&R.nstored, 1)) || (rc = dalloc(&R.scan_tmp, scan_tmp_entries(N))) ||
-        (rc = dalloc(&R.cell_gaps, cell_gap_entries(R.cell_cap))) || (rc = dalloc(&R.cell_ngap, 1)) ||
-        (rc = dalloc(&R.cell_start, R.cell_cap + 1)) || (rc = dalloc(&R.psort.keys, R.photon_cap)) ||
-        (rc = dalloc(&R.psort.vals, R.photon_cap)) || (rc = dalloc(&R.psort.tmp_k, R.photon_cap)) ||
-        (rc = dalloc(&R.psort.tmp_v, R.photon_cap)) || (rc = dalloc(&R.staged.rec, 3 * (size_t)R.photon_cap)) ||
-        (rc = dalloc(&R.psort.hist, radix_hist_entries(R.photon_cap))) ||
-        (rc = dalloc(&R.gpos, R.photon_cap)) || (rc = dalloc(&R.gflux, R.photon_cap)) ||
-        (rc = dalloc(&R.gdir, R.photon_cap)) || (rc = dalloc(&R.gp, 1)) || (rc = dalloc(&R.shared.rad, np)) ||
-        (rc = dalloc(&R.shared.cnt, np)) || (rc = dalloc(&R.shared.direct, np)) ||
-        (rc = dalloc(&R.counts, np + 1)) || (rc = dalloc(&R.list_off, np + 1)) ||
-        (rc = dalloc(&R.list_scan_tmp, scan_tmp_entries(np + 1))) ||
-        (rc = dalloc(&R.words, 2 * 6 * (size_t)np)) || (rc = dalloc(&R.cam_phi, MT_WORDS)) ||
-        (rc = dalloc(&R.rstat, 2)) || (rc = dalloc(&R.flags, 1)) || (rc = dalloc(&R.ctr, 1)) ||
-        (rc = dalloc(&R.raystripes, (size_t)STRIPES * RAY_STRIPE)) ||
-        (rc = dalloc((char**)&R.tiles, gather_tile_bytes() * (size_t)ntile_max)) ||
-        (rc = dalloc(&R.chunkp, 1)) || (rc = dalloc(&R.nch, ntile_max + 1)) ||
-        (rc = dalloc(&R.chunk_off, ntile_max + 1)) ||
-        (rc = dalloc(&R.tile_scan_tmp, scan_tmp_entries(ntile_max + 1))) ||
-        (rc = dalloc(&R.partial, (size_t)64 * (GATHER_CHUNK_CAP + ntile_max))) ||
-        (rc = dalloc(&R.groups.keys, np)) || (rc = dalloc(&R.groups.vals, np)) || (rc = dalloc(&R.groups.tmp_k, np)) ||
-        (rc = dalloc(&R.groups.tmp_v, np)) || (rc = dalloc(&R.groups.hist, radix_hist_entries(np))) ||
-        (rc = dalloc(&R.groups.nvalid, 1)) || (rc = dalloc(&R.groups.chunkq, STRIPE_INTS)) || (rc = dalloc(&R.groups.stat, 3 * (size_t)gather_group_count(np))) ||
-        (rc = dalloc(&R.groups.spheres, gather_sphere_entries(np))) ||
-        (rc = dalloc(&R.pass_dev, 3)) ||
-        (rc = dalloc(&R.image, np))) {
+    std::vector<long long> shape{N, W, Hh, c->params.photon_kernel, c->params.wave_bounces, c->params.wave_lanes,
+                                 c->scene.dev.width, c->scene.stack_cap, c->params.record_neighbours,
+                                 c->params.max_neighbours, c->cam.sampler == SPPM_SAMPLER_UNIFORM};
+    const bool keep = R.shape == shape;
+    if (!keep) {
         R.release();
-        return rc;
-    }
-    for (HitDev& h : R.hitbuf) {
-        if ((rc = dalloc(&h.pos, np)) || (rc = dalloc(&h.nrm, np)) || (rc = dalloc(&h.out, np)) ||
-            (rc = dalloc(&h.weight, np)) || (rc = dalloc(&h.mat, np)) || (rc = dalloc(&h.absorb, np)) ||
-            (rc = dalloc(&h.direct, np))) {
+        R.N = N; R.W = W; R.H = Hh; R.np = np;
+        // tiles of the recording gather (8x8 pixels) or hit-point groups of the production gather
+        const int ntile_max = std::max(gather_tile_count(W, Hh), gather_group_count(np));
+        R.slots.npaths = N;
+        if ((rc = dalloc(&R.slots.pos, NS)) || (rc = dalloc(&R.slots.flux, NS)) || (rc = dalloc(&R.slots.dir, NS)) ||
+            (rc = dalloc(&R.slots.valid, NS)) || (rc = dalloc(&R.slots.count, N)) || (rc = dalloc(&R.off, N)) ||
+            (rc = dalloc(&R.nstored, 1)) || (rc = dalloc(&R.scan_tmp, scan_tmp_entries(N))) ||
+            (rc = dalloc(&R.cell_gaps, cell_gap_entries(R.cell_cap))) || (rc = dalloc(&R.cell_ngap, 1)) ||
+            (rc = dalloc(&R.cell_start, R.cell_cap + 1)) || (rc = dalloc(&R.psort.keys, R.photon_cap)) ||
+            (rc = dalloc(&R.psort.vals, R.photon_cap)) || (rc = dalloc(&R.psort.tmp_k, R.photon_cap)) ||
+            (rc = dalloc(&R.psort.tmp_v, R.photon_cap)) || (rc = dalloc(&R.staged.rec, 3 * (size_t)R.photon_cap)) ||
+            (rc = dalloc(&R.psort.hist, radix_hist_entries(R.photon_cap))) ||
+            (rc = dalloc(&R.gpos, R.photon_cap)) || (rc = dalloc(&R.gflux, R.photon_cap)) ||
+            (rc = dalloc(&R.gdir, R.photon_cap)) || (rc = dalloc(&R.gp, 1)) || (rc = dalloc(&R.shared.rad, np)) ||
+            (rc = dalloc(&R.shared.cnt, np)) || (rc = dalloc(&R.shared.direct, np)) ||
+            (rc = dalloc(&R.counts, np + 1)) || (rc = dalloc(&R.list_off, np + 1)) ||
+            (rc = dalloc(&R.list_scan_tmp, scan_tmp_entries(np + 1))) ||
+            (rc = dalloc(&R.words, 2 * 6 * (size_t)np)) || (rc = dalloc(&R.cam_phi, MT_WORDS)) ||
+            (rc = dalloc(&R.rstat, 2)) || (rc = dalloc(&R.flags, 1)) || (rc = dalloc(&R.ctr, 1)) ||
+            (rc = dalloc(&R.raystripes, (size_t)STRIPES * RAY_STRIPE)) ||
+            (rc = dalloc((char**)&R.tiles, gather_tile_bytes() * (size_t)ntile_max)) ||
+            (rc = dalloc(&R.chunkp, 1)) || (rc = dalloc(&R.nch, ntile_max + 1)) ||
+            (rc = dalloc(&R.chunk_off, ntile_max + 1)) ||
+            (rc = dalloc(&R.tile_scan_tmp, scan_tmp_entries(ntile_max + 1))) ||
+            (rc = dalloc(&R.partial, (size_t)64 * (GATHER_CHUNK_CAP + ntile_max))) ||
+            (rc = dalloc(&R.groups.keys, np)) || (rc = dalloc(&R.groups.vals, np)) || (rc = dalloc(&R.groups.tmp_k, np)) ||
+            (rc = dalloc(&R.groups.tmp_v, np)) || (rc = dalloc(&R.groups.hist, radix_hist_entries(np))) ||
+            (rc = dalloc(&R.groups.nvalid, 1)) || (rc = dalloc(&R.groups.chunkq, STRIPE_INTS)) || (rc = dalloc(&R.groups.stat, 3 * (size_t)gather_group_count(np))) ||
+            (rc = dalloc(&R.groups.spheres, gather_sphere_entries(np))) ||
+            (rc = dalloc(&R.pass_dev, 3)) ||
+            (rc = dalloc(&R.image, np))) {
             R.release();
             return rc;
         }
-        h.np = np;
-    }
-    R.hits = R.hitbuf[0];
-    if (c->params.photon_kernel == SPPM_PHOTON_WAVEFRONT) {
-        const int B = c->params.wave_bounces > 0 ? c->params.wave_bounces : WAVE_BOUNCES_DEFAULT;
-        const int width = c->scene.dev.width;
-        int lanes = c->params.wave_lanes > 0 ? c->params.wave_lanes : WAVE_LANES_DEFAULT;
-        if (lanes > width) lanes = width;
-        if (!wave_lanes_ok(width, lanes)) {
-            R.release();
-            return fail(SPPM_E_ARG, "wave_lanes %d with a BVH of width %d", lanes, width);
+        for (HitDev& h : R.hitbuf) {
+            if ((rc = dalloc(&h.pos, np)) || (rc = dalloc(&h.nrm, np)) || (rc = dalloc(&h.out, np)) ||
+                (rc = dalloc(&h.weight, np)) || (rc = dalloc(&h.mat, np)) || (rc = dalloc(&h.absorb, np)) ||
+                (rc = dalloc(&h.direct, np))) {
+                R.release();
+                return rc;
+            }
+            h.np = np;
         }
-        R.wave_lanes = lanes;
-        R.wave_blocks = wave_trace_blocks(width, lanes);
-        if (R.wave_blocks <= 0) {
-            R.release();
-            return fail(SPPM_E_HIP, "cannot query the device for the trace kernel grid");
+        R.hits = R.hitbuf[0];
+        if (c->params.photon_kernel == SPPM_PHOTON_WAVEFRONT) {
+            const int B = c->params.wave_bounces > 0 ? c->params.wave_bounces : WAVE_BOUNCES_DEFAULT;
+            const int width = c->scene.dev.width;
+            int lanes = c->params.wave_lanes > 0 ? c->params.wave_lanes : WAVE_LANES_DEFAULT;
+            if (lanes > width) lanes = width;
+            if (!wave_lanes_ok(width, lanes)) {
+                R.release();
+                return fail(SPPM_E_ARG, "wave_lanes %d with a BVH of width %d", lanes, width);
+            }
+            R.wave_lanes = lanes;
+            R.wave_blocks = wave_trace_blocks(width, lanes);
+            if (R.wave_blocks <= 0) {
+                R.release();
+                return fail(SPPM_E_HIP, "cannot query the device for the trace kernel grid");
+            }
+            R.wave.cap = c->scene.stack_cap;
+            WaveBuffers& w = R.wave;
+            const size_t n = (size_t)N;
+            if ((rc = dalloc(&w.path.rng, n)) || (rc = dalloc(&w.path.org, n)) || (rc = dalloc(&w.path.dir, n)) ||
+                (rc = dalloc(&w.path.ndir, n)) || (rc = dalloc(&w.path.rad, n)) || (rc = dalloc(&w.path.thr, n)) ||
+                (rc = dalloc(&w.rays[0], 2 * wave_queue_entries(N))) ||
+                (rc = dalloc(&w.rays[1], 2 * wave_queue_entries(N))) || (rc = dalloc(&w.hits, wave_queue_entries(N))) ||
+                (rc = dalloc(&w.qctl, wave_ctl_ints(B))) ||
+                (rc = dalloc(&w.spill, wave_spill_entries(lanes, R.wave_blocks, R.wave.cap)))) {
+                R.release();
+                return rc;
+            }
+            R.wave_bounces = B;
         }
-        R.wave.cap = c->scene.stack_cap;
-        WaveBuffers& w = R.wave;
-        const size_t n = (size_t)N;
-        if ((rc = dalloc(&w.path.rng, n)) || (rc = dalloc(&w.path.org, n)) || (rc = dalloc(&w.path.dir, n)) ||
-            (rc = dalloc(&w.path.ndir, n)) || (rc = dalloc(&w.path.rad, n)) || (rc = dalloc(&w.path.thr, n)) ||
-            (rc = dalloc(&w.rays[0], 2 * wave_queue_entries(N))) ||
-            (rc = dalloc(&w.rays[1], 2 * wave_queue_entries(N))) || (rc = dalloc(&w.hits, wave_queue_entries(N))) ||
-            (rc = dalloc(&w.qctl, wave_ctl_ints(B))) ||
-            (rc = dalloc(&w.spill, wave_spill_entries(lanes, R.wave_blocks, R.wave.cap)))) {
-            R.release();
-            return rc;
+        if (c->params.record_neighbours == 2) {
+            R.pairs_cap = c->params.max_neighbours;
+            if ((rc = dalloc(&R.pairs, (size_t)R.pairs_cap)) || (rc = dalloc(&R.npairs, 2))) {
+                R.release();
+                return rc;
+            }
         }
-        R.wave_bounces = B;
-    }
-    if (c->params.record_neighbours == 2) {
-        R.pairs_cap = c->params.max_neighbours;
-        if ((rc = dalloc(&R.pairs, (size_t)R.pairs_cap)) || (rc = dalloc(&R.npairs, 2))) {
-            R.release();
-            return rc;
-        }
+        R.shape = std::move(shape);
     }
     if (c->guided) {
-        if ((rc = dalloc(&R.path_cell, 2 * (size_t)N)) || (rc = dalloc(&R.path_ratio, 2 * (size_t)N)) ||
-            (rc = dalloc(&R.pdep, R.photon_cap)) || (rc = dalloc(&R.doff, (size_t)N + 1))) {
+        if (!R.path_cell &&
+            ((rc = dalloc(&R.path_cell, 2 * (size_t)N)) || (rc = dalloc(&R.path_ratio, 2 * (size_t)N)) ||
+             (rc = dalloc(&R.pdep, R.photon_cap)) || (rc = dalloc(&R.doff, (size_t)N + 1)))) {
             R.release();
             return rc;
         }
         c->emit.path_cell = R.path_cell;
         c->emit.path_ratio = c->gparams.target == SPPM_GUIDE_TARGET_RMS ? R.path_ratio : nullptr;
+    } else {
+        dfree(R.path_cell); dfree(R.path_ratio); dfree(R.pdep); dfree(R.doff);
     }
     HIPOK(hipMemsetAsync(R.counts, 0, sizeof(int) * (size_t)(np + 1), c->stream));
     launch_init_slots(R.slots, c->stream);

@@ -13,6 +13,7 @@
 // sequence has P as its minimal polynomial.
 #include "sppm_mtjump.h"
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <stdexcept>
@@ -177,21 +178,28 @@ void mt_window_seed(uint32_t seed, uint32_t win[MT_WORDS]) {
     for (int i = 1; i < MT_WORDS; ++i) win[i] = 1812433253u * (win[i - 1] ^ (win[i - 1] >> 30)) + (uint32_t)i;
 }
 
+// The next 624 words in place.  Word i needs i, i + 1 and i + 397 (the word 227
+// before it in the new block, once that is made): three loops without a
+// remainder or a dependence closer than 227 words, which vectorise.
+static void next_block(uint32_t* __restrict__ x) {
+    const auto mix = [](uint32_t a, uint32_t b, uint32_t c) {
+        const uint32_t y = (a & MT_UPPER) | (b & MT_LOWER);
+        return c ^ (y >> 1) ^ ((0u - (y & 1u)) & MT_A);
+    };
+    for (int i = 0; i < 227; ++i) x[i] = mix(x[i], x[i + 1], x[i + 397]);
+    for (int i = 227; i < 454; ++i) x[i] = mix(x[i], x[i + 1], x[i - 227]);
+    for (int i = 454; i < 623; ++i) x[i] = mix(x[i], x[i + 1], x[i - 227]);
+    x[623] = mix(x[623], x[0], x[396]);
+}
+
 void mt_window_advance(uint32_t win[MT_WORDS], uint64_t steps) {
-    // ring of the window; head = oldest word
-    uint32_t ring[MT_WORDS];
-    for (int i = 0; i < MT_WORDS; ++i) ring[i] = win[i];
-    unsigned head = 0;
-    for (uint64_t s = 0; s < steps; ++s) {
-        const unsigned i1 = head + 1 == MT_WORDS ? 0 : head + 1;
-        const unsigned i397 = head + 397 >= MT_WORDS ? head + 397 - MT_WORDS : head + 397;
-        ring[head] = mt_mix(ring[head], ring[i1], ring[i397]);
-        head = i1;
-    }
-    for (int i = 0; i < MT_WORDS; ++i) {
-        const unsigned k = head + i >= MT_WORDS ? head + i - MT_WORDS : head + i;
-        win[i] = ring[k];
-    }
+    for (; steps >= MT_WORDS; steps -= MT_WORDS) next_block(win);
+    if (steps == 0) return;
+    uint32_t next[MT_WORDS];
+    std::copy(win, win + MT_WORDS, next);
+    next_block(next);
+    std::copy(win + steps, win + MT_WORDS, win);
+    std::copy(next, next + steps, win + MT_WORDS - steps);
 }
 
 void mt_jump_poly(uint64_t J, uint32_t phi[MT_WORDS]) {

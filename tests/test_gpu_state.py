@@ -112,3 +112,48 @@ def test_checkpoint_refuses_other_setups(box_scene):
         np.testing.assert_array_equal(a[k], b[k])
     r.close()
     same.close()
+
+
+@pytest.mark.parametrize("change", ["same", "sampler", "alpha", "scene", "guided", "size", "graph"])
+def test_begin_again_equals_fresh(change, box_scene):
+    """sppm_begin keeps the buffers of a render of the same sizes: after passes
+    that filled them, the next render equals one from a new context, with the
+    same setup or with one part of it changed."""
+    cam = scenes.pinhole_camera(40, 24)
+    guide = dict(learning_rate=1e-3, train_steps=1)
+    other = scenes.transmit_scene() if change == "scene" else box_scene
+    cam2 = dict(cam, sampler=sppm_amd.SAMPLER_HALTON) if change == "sampler" else cam
+    if change == "size":
+        cam2 = scenes.pinhole_camera(41, 24)
+    alpha = 0.7 if change == "alpha" else 0.9
+
+    def render(r):
+        if change == "graph":
+            r.graph_capture()
+        for _ in range(3):
+            r.pass_(stats=False)
+        sh = r.read_shared()
+        return [r.reconstruct()] + [sh[k] for k in sorted(sh)]
+
+    r = sppm_amd.Renderer(box_scene, cam, 0.9, 0.05, 6000, bvh_width=4)
+    if change == "guided":
+        r.guide_set(True, **guide)
+        r.begin()
+    for _ in range(4):
+        r.pass_(stats=False)
+    r.upload_scene(other, 4)
+    r._cam = sppm_amd.camera_desc(cam2)
+    sppm_amd._check(r.lib.sppm_camera_set(r.h, sppm_amd.C.byref(r._cam)))
+    r.W, r.H = cam2["width"], cam2["height"]
+    r._params = sppm_amd.params_struct(alpha, 0.05, 6000, 4, False)
+    sppm_amd._check(r.lib.sppm_params_set(r.h, sppm_amd.C.byref(r._params)))
+    if change == "guided":
+        r.guide_set(False)
+    r.begin()
+    again = render(r)
+    r.close()
+    f = sppm_amd.Renderer(other, cam2, alpha, 0.05, 6000, bvh_width=4)
+    fresh = render(f)
+    f.close()
+    for a, b in zip(again, fresh):
+        np.testing.assert_array_equal(a, b)
