@@ -1209,9 +1209,18 @@ __device__ __forceinline__ RowSpan group_rows(const TileRange& T, int ny, int nr
     return s;
 }
 
-// Per group: its union cell box, its candidate count, and its hit points'
-// query spheres (centre, squared radius; -1: no hit point) for the chunk
-// kernel's scalar loads.
+// A group's query spheres, for the chunk kernel's scalar loads: centre and
+// squared radius of each hit point (-1: no hit point); then the same about the
+// group's centre o as (-2 (c - o), |c - o|^2 - R^2), with which a photon's
+// squared distance minus R^2 is three FMAs; then o and the largest
+// |c - o|^2 + R^2 (-1: the group is wide for its radii, use the first form).
+constexpr int SPHERES = 2 * GATHER_GROUP + 1;
+// Error of the second form against the first, per |p - o|^2 + that largest
+// value: (p - c)^2 in float32, both centred positions (half an ulp each), the
+// two squares and the six sums are at most 21 roundings of terms that are no
+// larger than (|p - o| + |c - o|)^2 + R^2, twice that sum at most: 42 * 2^-24.
+constexpr float SPHERE_MARGIN = 0x1p-18f;
+// Per group: its union cell box, its candidate count and its query spheres.
 __global__ void __launch_bounds__(64) k_gather_plan(HitDev H, SharedDev SH, GridDev G, const GridParams* __restrict__ gp,
                                                     const uint32_t* __restrict__ order, const int* __restrict__ nvalidp,
                                                     TileRange* __restrict__ tiles, float4* __restrict__ spheres) {
@@ -1223,8 +1232,23 @@ __global__ void __launch_bounds__(64) k_gather_plan(HitDev H, SharedDev SH, Grid
     float4 sr;
     int r[6];
     load_gather_lane(H, SH, g, p, L, active, sr, r);
-    if (lane < GATHER_GROUP)
-        spheres[(size_t)blockIdx.x * GATHER_GROUP + lane] = make_float4(L.c.x, L.c.y, L.c.z, active ? L.R2 : -1.0f);
+    {
+        const bool in = active && L.R2 >= 0.0f;
+        const float BIG = 3.0e38f;
+        const f3 o = mk((wave_min(in ? L.c.x : BIG) + wave_max(in ? L.c.x : -BIG)) * 0.5f,
+                        (wave_min(in ? L.c.y : BIG) + wave_max(in ? L.c.y : -BIG)) * 0.5f,
+                        (wave_min(in ? L.c.z : BIG) + wave_max(in ? L.c.z : -BIG)) * 0.5f);
+        const f3 c = L.c - o;
+        const float cc = norm2(c);
+        const float far = wave_max(in ? cc + L.R2 : 0.0f), rmin = wave_min(in ? L.R2 : BIG);
+        float4* const sp = spheres + (size_t)blockIdx.x * SPHERES;
+        if (lane < GATHER_GROUP) {
+            sp[lane] = make_float4(L.c.x, L.c.y, L.c.z, active ? L.R2 : -1.0f);
+            sp[GATHER_GROUP + lane] =
+                in ? make_float4(-2.0f * c.x, -2.0f * c.y, -2.0f * c.z, cc - L.R2) : make_float4(0.0f, 0.0f, 0.0f, BIG);
+        }
+        if (lane == 0) sp[2 * GATHER_GROUP] = make_float4(o.x, o.y, o.z, far < 1e30f && far < 512.0f * rmin ? far : -1.0f);
+    }
     TileRange T;
     T.x0 = -wave_max_i(active ? -r[0] : -0x7fffffff); T.x1 = wave_max_i(active ? r[1] : -1);
     T.y0 = -wave_max_i(active ? -r[2] : -0x7fffffff); T.y1 = wave_max_i(active ? r[3] : -1);
@@ -1303,8 +1327,10 @@ __device__ __forceinline__ uint32_t transpose32(uint32_t x, int lane) {
 // its chunk at a time, one per lane, filled across the rows of the group's
 // box, and tests them against the group's hit points one after the other:
 // the hit point's centre and squared radius are scalars (scalar loads), so a
-// test is nine vector instructions for 64 pairs and one or two to keep its
-// bit.  The bits are transposed from masks per photon to masks per hit point
+// test is six vector instructions for 64 pairs about the group's centre (a sum,
+// three FMAs, the sign into the mask, the smallest magnitude), and where a
+// result is within its rounding error of zero, or the group is wide for its
+// radii, the exact form's ten for the batch.  The bits are transposed from masks per photon to masks per hit point
 // (five exchange steps), and every lane walks the set bits of its mask and accumulates BRDF * Flux / PDF (SPPM.cpp:434-440), in ascending
 // candidate order; the photons' directions and fluxes are in LDS.
 //
@@ -1314,14 +1340,15 @@ __device__ __forceinline__ uint32_t transpose32(uint32_t x, int lane) {
 // monotonic), so fl(p - c)^2 >= fl(R * R) and the sum of squares is no less;
 // the upper sides alike, and with NaN both tests fail.
 //
-// Bound by vector instructions: about 10 per 64 pairs tested and 25 to 60 per
+// Bound by vector instructions: about 6 per 64 pairs tested and 25 to 60 per
 // neighbour.  Before, a lane tested staged photons from LDS (22 instructions
 // and a 16-byte LDS read per pair, one row of cells at a time) over the whole
 // union box; a wave that entered a wide group walked its rows one dependent
 // load at a time.  The gather alone, mean of a render's first 8 passes: 64^2
 // pixels and 5k photons 0.504 -> 0.191 ms, 256^2 and 100k 0.688 -> 0.228,
 // 1024^2 and 1M (203k triangles) 2.715 -> 1.92, 1024^2 and 4M (caustics)
-// 12.76 -> 3.72.
+// 12.76 -> 3.72; with the sum of FMAs 1.87 -> 1.80 and 3.12 -> 3.01 (1M and 4M
+// again).
 // The chunks of one scene's gather, claimed until its counters are exhausted.
 __device__ __forceinline__ void gather_chunks(HitDev H, SharedDev SH, GridDev G,
                                               const GridParams* __restrict__ gp, const uint32_t* __restrict__ order,
@@ -1361,7 +1388,8 @@ __device__ __forceinline__ void gather_chunks(HitDev H, SharedDev SH, GridDev G,
         // constant address space: scalar loads also where the pointer comes from a job table
         typedef float sphere_t __attribute__((ext_vector_type(4)));
         typedef const sphere_t __attribute__((address_space(4))) * sphere_ptr;
-        const sphere_ptr sph = (sphere_ptr)(uintptr_t)(spheres + (size_t)t * GATHER_GROUP);
+        const sphere_ptr sph = (sphere_ptr)(uintptr_t)(spheres + (size_t)t * SPHERES);
+        const sphere_t so = sph[2 * GATHER_GROUP];
         const int p = group_pixel(order, nvalid, t * GATHER_GROUP + hl);
         GatherLane L;
         bool active;
@@ -1412,10 +1440,30 @@ __device__ __forceinline__ void gather_chunks(HitDev H, SharedDev SH, GridDev G,
                 uint32_t mask = 0;  // bit i: hit point i gathers this lane's photon
                 // lanes past n hold no candidate
                 const f3 pos = mk(lane < n ? pp.x : __builtin_inff(), pp.y, pp.z);
+                bool sure = so.w >= 0.0f;
+                if (sure) {
+                    f3 c = mk(pp.x - so.x, pp.y - so.y, pp.z - so.z);
+                    float cc = norm2(c);
+                    if (!(lane < n && cc < 1e37f)) {  // far beyond every sphere, or no position
+                        c = mk(0.0f, 0.0f, 0.0f);
+                        cc = 3.0e38f;
+                    }
+                    float least = 3.0e38f;
 #pragma unroll 16
-                for (int i = GATHER_GROUP - 1; i >= 0; --i) {
-                    const sphere_t sp = sph[i];
-                    mask = (mask << 1) + (norm2(pos - mk(sp.x, sp.y, sp.z)) < sp.w ? 1u : 0u);
+                    for (int i = GATHER_GROUP - 1; i >= 0; --i) {
+                        const sphere_t sp = sph[GATHER_GROUP + i];
+                        const float e = __builtin_fmaf(c.z, sp.z, __builtin_fmaf(c.y, sp.y, __builtin_fmaf(c.x, sp.x, cc + sp.w)));
+                        mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(e), 31);  // mask << 1 | sign
+                        least = fminf(least, fabs_(e));
+                    }
+                    sure = __ballot(least < SPHERE_MARGIN * (cc + so.w)) == 0ull;
+                }
+                if (!sure) {
+#pragma unroll 16
+                    for (int i = GATHER_GROUP - 1; i >= 0; --i) {
+                        const sphere_t sp = sph[i];
+                        mask = (mask << 1) + (norm2(pos - mk(sp.x, sp.y, sp.z)) < sp.w ? 1u : 0u);
+                    }
                 }
                 const int cnt = __popc(mask);  // hit points of the group that gather this lane's photon
                 mask = transpose32(mask, lane);  // bit j: staged photon ph * 32 + j is gathered by this lane's hit point
@@ -1953,7 +2001,7 @@ const uint32_t* gather_order(const GroupBuffers& gb, int np) {
 }
 int gather_tile_count(int W, int Hh) { return ((W + 7) >> 3) * ((Hh + 7) >> 3); }
 int gather_group_count(int np) { return (np + GATHER_GROUP - 1) / GATHER_GROUP; }
-size_t gather_sphere_entries(int np) { return (size_t)gather_group_count(np) * GATHER_GROUP; }
+size_t gather_sphere_entries(int np) { return (size_t)gather_group_count(np) * SPHERES; }
 size_t gather_tile_bytes() { return sizeof(TileRange); }
 
 void launch_reconstruct(const SharedDev& SH, int np, long long total, int passes, float4* out, hipStream_t st) {
