@@ -144,9 +144,7 @@ struct RenderBuffers {
     TileRange* tiles = nullptr;
     int ntiles = 0;
     int* chunkp = nullptr;
-    int* nch = nullptr;
     int* chunk_off = nullptr;
-    int* tile_scan_tmp = nullptr;
     float4* partial = nullptr;
     GroupBuffers groups{};
     int* pass_dev = nullptr;   // passes done (device copy of the pass counter, read by graph replays);
@@ -192,7 +190,7 @@ struct RenderBuffers {
         }
         hits = HitDev{};
         dfree(shared.rad); dfree(shared.cnt); dfree(shared.direct); dfree(counts); dfree(list_off); dfree(list_scan_tmp); dfree(lists);
-        dfree(words); dfree(cam_states); dfree(cam_phi); dfree(rstat); dfree(tiles); dfree(chunkp); dfree(nch); dfree(chunk_off); dfree(tile_scan_tmp); dfree(partial); dfree(groups.keys); dfree(groups.vals); dfree(groups.tmp_k); dfree(groups.tmp_v); dfree(groups.hist); dfree(groups.nvalid); dfree(groups.chunkq); dfree(groups.stat); dfree(groups.spheres); dfree(pass_dev); dfree(path_cell); dfree(path_ratio); dfree(pdep); dfree(doff); dfree(flags); dfree(ctr); dfree(raystripes); dfree(image);
+        dfree(words); dfree(cam_states); dfree(cam_phi); dfree(rstat); dfree(tiles); dfree(chunkp); dfree(chunk_off); dfree(partial); dfree(groups.keys); dfree(groups.vals); dfree(groups.tmp_k); dfree(groups.tmp_v); dfree(groups.hist); dfree(groups.nvalid); dfree(groups.chunkq); dfree(groups.stat); dfree(groups.spheres); dfree(pass_dev); dfree(path_cell); dfree(path_ratio); dfree(pdep); dfree(doff); dfree(flags); dfree(ctr); dfree(raystripes); dfree(image);
         lists_cap = 0;
         shape.clear();
         ready = false;
@@ -1038,9 +1036,8 @@ int sppm_begin(sppm_ctx* c) {
             (rc = dalloc(&R.rstat, 2)) || (rc = dalloc(&R.flags, 1)) || (rc = dalloc(&R.ctr, 1)) ||
             (rc = dalloc(&R.raystripes, (size_t)STRIPES * RAY_STRIPE)) ||
             (rc = dalloc((char**)&R.tiles, gather_tile_bytes() * (size_t)ntile_max)) ||
-            (rc = dalloc(&R.chunkp, 1)) || (rc = dalloc(&R.nch, ntile_max + 1)) ||
+            (rc = dalloc(&R.chunkp, 1)) ||
             (rc = dalloc(&R.chunk_off, ntile_max + 1)) ||
-            (rc = dalloc(&R.tile_scan_tmp, scan_tmp_entries(ntile_max + 1))) ||
             (rc = dalloc(&R.partial, (size_t)64 * (GATHER_CHUNK_CAP + ntile_max))) ||
             (rc = dalloc(&R.groups.keys, np)) || (rc = dalloc(&R.groups.vals, np)) || (rc = dalloc(&R.groups.tmp_k, np)) ||
             (rc = dalloc(&R.groups.tmp_v, np)) || (rc = dalloc(&R.groups.hist, radix_hist_entries(np))) ||
@@ -1350,11 +1347,10 @@ static int do_gather(sppm_ctx* c, hipStream_t st) {
                       R.ctr, R.flags, st);
         R.have_lists = true;
     } else {
-        launch_set_u64x2(R.rstat, 0ull, 0ull, st);
         if (c->guided) launch_deposit_clear(R.pdep, R.doff + R.N, st);
         const PairRecord rec{R.pairs, R.npairs, R.pairs_cap};
         launch_gather_balanced(R.hits, R.shared, G, R.gp, R.np, c->scene.bmin, c->scene.ext, R.groups, alpha, R.tiles,
-                               GATHER_CHUNK_CAP, R.chunkp, R.nch, R.chunk_off, R.tile_scan_tmp, R.partial, R.counts,
+                               GATHER_CHUNK_CAP, R.chunkp, R.chunk_off, R.partial, R.counts,
                                R.rstat, R.ctr, R.flags, c->guided ? R.pdep : nullptr, rec, st);
         R.have_lists = R.pairs != nullptr;
     }
@@ -2033,11 +2029,10 @@ static int enqueue_multi(sppm_batch* b, hipStream_t st) {
     r = batch_branches(b, st, [&](int k, hipStream_t bs) {
         sppm_ctx* c = b->ctx[k];
         RenderBuffers& R = c->rb;
-        launch_set_u64x2(R.rstat, 0ull, 0ull, bs);
         if (c->guided) launch_deposit_clear(R.pdep, R.doff + R.N, bs);
         const PairRecord rec{R.pairs, R.npairs, R.pairs_cap};
         (void)launch_gather_plan(R.hits, R.shared, grid_dev(c), R.gp, R.np, c->scene.bmin, c->scene.ext, R.groups,
-                                 R.tiles, GATHER_CHUNK_CAP, R.chunkp, R.nch, R.chunk_off, R.tile_scan_tmp, R.counts,
+                                 R.tiles, GATHER_CHUNK_CAP, R.chunkp, R.chunk_off, R.counts,
                                  R.ctr, rec, bs);
     });
     if (r) return r;

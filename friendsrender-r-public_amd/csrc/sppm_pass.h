@@ -141,7 +141,7 @@ struct PairRecord {
 };
 void launch_gather_balanced(const HitDev& H, const SharedDev& SH, const GridDev& G, const GridParams* gp, int np,
                             const float* bmin, const float* ext, const GroupBuffers& gb, float alpha, TileRange* tiles,
-                            int cap, int* chunkp, int* nch, int* chunk_off, int* scan_tmp, float4* partial,
+                            int cap, int* chunkp, int* chunk_off, float4* partial,
                             int* counts, unsigned long long* rstat, Counters* ctr, uint32_t* flags,
                             unsigned long long* pdep,
                             const PairRecord& rec, hipStream_t st);
@@ -149,7 +149,7 @@ void launch_gather_balanced(const HitDev& H, const SharedDev& SH, const GridDev&
 // returns the group order), the chunk kernel, and the per-group sums.
 const uint32_t* launch_gather_plan(const HitDev& H, const SharedDev& SH, const GridDev& G, const GridParams* gp,
                                    int np, const float* bmin, const float* ext, const GroupBuffers& gb,
-                                   TileRange* tiles, int cap, int* chunkp, int* nch, int* chunk_off, int* scan_tmp,
+                                   TileRange* tiles, int cap, int* chunkp, int* chunk_off,
                                    int* counts, Counters* ctr, const PairRecord& rec, hipStream_t st);
 void launch_gather_run(const HitDev& H, const SharedDev& SH, const GridDev& G, const GridParams* gp, int np,
                        const uint32_t* order, const GroupBuffers& gb, const TileRange* tiles, const int* chunkp,

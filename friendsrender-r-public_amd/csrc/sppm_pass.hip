@@ -1057,9 +1057,8 @@ __global__ void __launch_bounds__(64) k_gather(HitDev H, SharedDev SH, GridDev G
 // Candidate counts per 8x8 tile vary by orders of magnitude (caustics), so:
 //   k_gather_plan    per tile: union cell box of its hit points, the
 //                    candidates of its rows (group_rows) and the query spheres
-//   k_chunk_size     candidates per chunk so that all chunks fit the buffer
-//   k_tile_chunks    chunks per tile
-//   scan             chunk offsets per tile
+//   k_chunks         candidates per chunk so that all chunks fit the buffer,
+//                    and every tile's chunk offset
 //   k_gather_chunks  persistent waves take chunks of one tile's candidates
 //                    and write per-lane partial sums
 //   k_gather_finish  per tile: partial sums in chunk order + the update
@@ -1095,8 +1094,10 @@ __device__ __forceinline__ int quant10(float p, float lo, float ext) {
 }
 constexpr uint32_t HIT_KEY_INVALID = 1u << 30;  // above every 30-bit Morton code: invalid hit points sort last
 __global__ void k_hit_keys(HitDev H, int np, float bx, float by, float bz, float ex, float ey, float ez,
-                           uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+                           uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, int* __restrict__ chunkq) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    // the chunk kernel's counters, a few launches later
+    for (int k = i; k < STRIPE_INTS; k += gridDim.x * blockDim.x) chunkq[k] = 0;
     if (i >= np) return;
     const float4 hp = H.pos[i];
     uint32_t key = HIT_KEY_INVALID;
@@ -1274,33 +1275,52 @@ __global__ void __launch_bounds__(64) k_gather_plan(HitDev H, SharedDev SH, Grid
 // their buffer (cap).  Always 1024 left a pass of few candidates on a few
 // hundred waves.
 constexpr int GATHER_CHUNKS_PER_WAVE = 2;
-__global__ void __launch_bounds__(256) k_chunk_size(const TileRange* __restrict__ tiles, int ntiles, int cap,
-                                                    int* __restrict__ chunk, Counters* __restrict__ ctr) {
-    __shared__ unsigned long long part[4];
+// One workgroup makes the chunk size, every group's chunk count and their
+// offsets (chunk_off[ntiles]: all chunks): six short launches before, whose
+// own 4 to 5 us each were a tenth of a small render's pass.
+constexpr int CHUNK_THREADS = 1024;
+__global__ void __launch_bounds__(CHUNK_THREADS) k_chunks(const TileRange* __restrict__ tiles, int ntiles, int cap,
+                                                          int* __restrict__ chunk, int* __restrict__ chunk_off,
+                                                          Counters* __restrict__ ctr) {
+    __shared__ unsigned long long part[CHUNK_THREADS / 64];
+    __shared__ int wsum[CHUNK_THREADS / 64], sh_chunk;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int per = (ntiles + CHUNK_THREADS - 1) / CHUNK_THREADS;
+    const int t0 = min((int)threadIdx.x * per, ntiles), t1 = min(t0 + per, ntiles);
     unsigned long long s = 0;
-    for (int t = threadIdx.x; t < ntiles; t += 256) s += (unsigned long long)tiles[t].cand;
+    for (int t = t0; t < t1; ++t) s += (unsigned long long)tiles[t].cand;
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+    if (lane == 0) part[wave] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
-        unsigned long long tot = part[0] + part[1] + part[2] + part[3];
+        unsigned long long tot = 0;
+        for (int w = 0; w < CHUNK_THREADS / 64; ++w) tot += part[w];
         unsigned long long c = (tot + (unsigned long long)cap - 1) / (unsigned long long)cap;
         unsigned long long lo = tot / (unsigned long long)(GATHER_WAVES * GATHER_CHUNKS_PER_WAVE);
         lo = lo < 128 ? 128 : lo > 1024 ? 1024 : lo;
         if (c < lo) c = lo;
         c = (c + 63) & ~63ull;
-        *chunk = (int)c;
+        *chunk = sh_chunk = (int)c;
         ctr->candidates += tot;
     }
-}
-
-__global__ void k_tile_chunks(const TileRange* __restrict__ tiles, int ntiles, const int* __restrict__ chunk,
-                              int* __restrict__ nch) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t > ntiles) return;
-    if (t == ntiles) { nch[t] = 0; return; }
-    const int c = *chunk;
-    nch[t] = (tiles[t].cand + c - 1) / c;
+    __syncthreads();
+    const int c = sh_chunk;
+    int n = 0;
+    for (int t = t0; t < t1; ++t) n += (tiles[t].cand + c - 1) / c;
+    int incl = n;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += v;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int run = incl - n;
+    for (int w = 0; w < wave; ++w) run += wsum[w];
+    for (int t = t0; t < t1; ++t) {
+        chunk_off[t] = run;
+        run += (tiles[t].cand + c - 1) / c;
+    }
+    if (threadIdx.x == CHUNK_THREADS - 1) chunk_off[ntiles] = run;
 }
 
 // Transposes the 32 x 32 bit matrix that each half of the wave holds, a row
@@ -1656,8 +1676,8 @@ __global__ void __launch_bounds__(1024) k_group_stats(const unsigned long long* 
             b += part[1][k];
             c += part[2][k];
         }
-        rstat[0] += a;
-        rstat[1] += b;
+        rstat[0] = a;
+        rstat[1] = b;
         ctr->hit_points += b;
         ctr->neighbours += c;
     }
@@ -1916,22 +1936,18 @@ void launch_gather(const HitDev& H, const SharedDev& SH, const GridDev& G, const
 
 const uint32_t* launch_gather_plan(const HitDev& H, const SharedDev& SH, const GridDev& G, const GridParams* gp,
                                    int np, const float* bmin, const float* ext, const GroupBuffers& gb,
-                                   TileRange* tiles, int cap, int* chunkp, int* nch, int* chunk_off, int* scan_tmp,
+                                   TileRange* tiles, int cap, int* chunkp, int* chunk_off,
                                    int* counts, Counters* ctr, const PairRecord& rec, hipStream_t st) {
     const int ntiles = gather_group_count(np);
     // hit-point groups: valid hit points in Morton order, GATHER_GROUP per group
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, st, gb.nvalid, 1);  // valid count
-    hipLaunchKernelGGL(k_zero_i32, dim3(STRIPE_INTS / 256), dim3(256), 0, st, gb.chunkq, STRIPE_INTS);
     if (counts) hipLaunchKernelGGL(k_zero_i32, dim3((np + 255) / 256), dim3(256), 0, st, counts, np);
     hipLaunchKernelGGL(k_hit_keys, dim3((np + 255) / 256), dim3(256), 0, st, H, np, bmin[0], bmin[1], bmin[2], ext[0],
-                       ext[1], ext[2], gb.keys, gb.vals);
+                       ext[1], ext[2], gb.keys, gb.vals, gb.chunkq);
     const SortResult sr = radix_sort_pairs(gb.keys, gb.vals, gb.tmp_k, gb.tmp_v, gb.hist, np, 31, st);
     hipLaunchKernelGGL(k_count_valid, dim3(1), dim3(64), 0, st, sr.keys, np, gb.nvalid);
     const uint32_t* order = sr.vals;  // == gather_order(gb, np)
     hipLaunchKernelGGL(k_gather_plan, dim3(ntiles), dim3(64), 0, st, H, SH, G, gp, order, gb.nvalid, tiles, gb.spheres);
-    hipLaunchKernelGGL(k_chunk_size, dim3(1), dim3(256), 0, st, tiles, ntiles, cap, chunkp, ctr);
-    hipLaunchKernelGGL(k_tile_chunks, dim3((ntiles + 1 + 255) / 256), dim3(256), 0, st, tiles, ntiles, chunkp, nch);
-    exclusive_scan(nch, chunk_off, ntiles + 1, nullptr, scan_tmp, st);
+    hipLaunchKernelGGL(k_chunks, dim3(1), dim3(CHUNK_THREADS), 0, st, tiles, ntiles, cap, chunkp, chunk_off, ctr);
     if (rec.pairs) launch_set_u64x2(rec.count, 0ull, 0ull, st);
     return order;
 }
@@ -1952,12 +1968,12 @@ void launch_gather_finish(const HitDev& H, const SharedDev& SH, int np, const ui
 }
 void launch_gather_balanced(const HitDev& H, const SharedDev& SH, const GridDev& G, const GridParams* gp, int np,
                             const float* bmin, const float* ext, const GroupBuffers& gb, float alpha, TileRange* tiles,
-                            int cap, int* chunkp, int* nch, int* chunk_off, int* scan_tmp, float4* partial,
+                            int cap, int* chunkp, int* chunk_off, float4* partial,
                             int* counts, unsigned long long* rstat, Counters* ctr, uint32_t* flags,
                             unsigned long long* pdep,
                             const PairRecord& rec, hipStream_t st) {
-    const uint32_t* order = launch_gather_plan(H, SH, G, gp, np, bmin, ext, gb, tiles, cap, chunkp, nch, chunk_off,
-                                               scan_tmp, counts, ctr, rec, st);
+    const uint32_t* order = launch_gather_plan(H, SH, G, gp, np, bmin, ext, gb, tiles, cap, chunkp, chunk_off,
+                                               counts, ctr, rec, st);
     launch_gather_run(H, SH, G, gp, np, order, gb, tiles, chunkp, chunk_off, partial, pdep, rec, st);
     launch_gather_finish(H, SH, np, order, gb, alpha, chunk_off, partial, counts, rstat, ctr, flags, st);
 }

@@ -322,6 +322,18 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(const int* __restri
     }
     if (threadIdx.x == 0) tile_sums[blockIdx.x] = tot;
 }
+// out += the sums of the tiles before (each workgroup adds them up itself).
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_carry(int* __restrict__ out, int n,
+                                                             const int* __restrict__ tile_sums, int* __restrict__ total,
+                                                             int ntiles) {
+    int s = 0, add;
+    for (int j = threadIdx.x; j < (int)blockIdx.x; j += SCAN_THREADS) s += tile_sums[j];
+    block_excl_scan(s, &add);
+    const int base = blockIdx.x * SCAN_TILE;
+    for (int i = threadIdx.x; i < SCAN_TILE; i += SCAN_THREADS)
+        if (base + i < n) out[base + i] += add;
+    if (blockIdx.x == ntiles - 1 && threadIdx.x == 0 && total) *total = add + tile_sums[ntiles - 1];
+}
 __global__ void __launch_bounds__(SCAN_THREADS) k_scan_add(int* __restrict__ out, int n,
                                                            const int* __restrict__ tile_pre, int* __restrict__ total,
                                                            int ntiles) {
@@ -338,10 +350,18 @@ size_t scan_tmp_entries(int n) {
     int nt = (n + SCAN_TILE - 1) / SCAN_TILE;
     return (size_t)nt + 1 + 64;
 }
+// Up to this many tiles (4M items) each adds up the sums before it, 4 KB to
+// read on average; beyond, they are scanned first, in two more launches of
+// about 5 us each.
+constexpr int SCAN_CARRY_TILES = 2048;
 void exclusive_scan(const int* in, int* out, int n, int* total, int* tmp, hipStream_t st) {
     if (n <= 0) return;
     int nt = (n + SCAN_TILE - 1) / SCAN_TILE;
     hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(SCAN_THREADS), 0, st, in, out, n, tmp);
+    if (nt <= SCAN_CARRY_TILES) {
+        hipLaunchKernelGGL(k_scan_carry, dim3(nt), dim3(SCAN_THREADS), 0, st, out, n, tmp, total, nt);
+        return;
+    }
     // tile sums -> exclusive prefix with total in tmp[nt] (nt tiles fit one small scan)
     hipLaunchKernelGGL(k_tile_total_prep, dim3(1), dim3(1), 0, st, tmp, nt);
     hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(1024), 0, st, reinterpret_cast<uint32_t*>(tmp), nt + 1);

@@ -55,3 +55,14 @@ def test_grid_layout_full_workload():
         r.pass_(stats=False)
         check_grid(r, f"full-material pass {p + 1}")
     r.close()
+
+
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 4194304, 4194305])
+def test_photon_offsets_scan_sizes(n, box_scene):
+    """The stored photons of path counts around a scan tile (2048) and around
+    the tile count where the scan of the tile sums becomes a launch of its own."""
+    r = sppm_amd.Renderer(box_scene, scenes.pinhole_camera(8, 8), 0.9, 0.015, n, bvh_width=8)
+    r.photons(1)
+    stored = r.build()
+    assert stored == int(r.read_path_counts().astype(np.int64).sum())
+    r.close()
