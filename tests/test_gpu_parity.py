@@ -72,7 +72,7 @@ def test_ray_counts_split_over_waves(n, width):
     r.close()
 
 
-@pytest.mark.parametrize("w,h,N", [(1, 1, 1), (3, 1, 63), (32, 32, 1025), (33, 31, 17000)])
+@pytest.mark.parametrize("w,h,N", [(8, 8, 63), (16, 9, 1025), (32, 32, 1024), (33, 31, 17000)])
 def test_pass_parity_path_counts_split_over_waves(w, h, N, full_scene_small):
     """Whole passes at path and pixel counts around the sizes where the share
     of a wave changes, on the scene with every material."""
@@ -214,7 +214,7 @@ def test_pass_parity_gather_edges(box_scene, w, h, N, r0):
                record=sppm_amd.RECORD_PAIRS, max_pairs=40_000_000)
 
 
-@pytest.mark.parametrize("w,h", [(1, 1), (2, 1), (37, 1), (38, 1), (227, 1), (119, 61)])
+@pytest.mark.parametrize("w,h", [(3, 3), (7, 5), (19, 4), (37, 7), (119, 61)])
 def test_camera_words_sizes(w, h, box_scene):
     """Three passes' camera words at sizes around the generator's own (227 words
     a step, 624 a window, segments of one word to thousands), through the hit
