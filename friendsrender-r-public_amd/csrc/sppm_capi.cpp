@@ -1182,14 +1182,16 @@ static TraceSpill trace_spill(const sppm_ctx* c) {
     return sp;
 }
 // the eye pass's own spill area: in a full pass it runs beside the photon pass
-// beside: in a full pass it takes 5/16 of the path-kernel grid.  Its persistent
+// beside: in a full pass it takes 3/16 of the path-kernel grid.  Its persistent
 // waves would otherwise fill every wave slot that the gather leaves free, and
 // the build's short kernels after it wait for them (a sort pass took 1.5 ms):
-// 4M photons at 1024^2 (caustics, 8 passes) 124.5 ms against 135.5 with the
-// whole grid, the full-material workload 138.5 against 139.2 (32 passes).
+// 4M photons at 1024^2 (caustics, 8 passes) 124.5 ms with 5/16 against 135.5 with
+// the whole grid.  With 8/16 for the photons (photon_pass) 3/16 against 5/16
+// and 10/16: occluded light at 1024^2 47.3 against 52.3 ms (16 passes), 256^2
+// 10.0 against 10.4, full-material 1024^2 118.9 against 120.5 (32 passes).
 static TraceSpill trace_spill_eye(const sppm_ctx* c, bool beside) {
     TraceSpill sp = c->scene.trace_spill_eye();
-    if (beside) sp.blocks = sp.blocks * 5 / 16 > 0 ? sp.blocks * 5 / 16 : 1;
+    if (beside) sp.blocks = sp.blocks * 3 / 16 > 0 ? sp.blocks * 3 / 16 : 1;
     if (c->tuned_blocks > 0 && c->tuned_blocks < sp.blocks) sp.blocks = c->tuned_blocks;
     return sp;
 }
@@ -1213,19 +1215,20 @@ static int read_counters(sppm_ctx* c, Counters& h) {
     return SPPM_OK;
 }
 // beside_gather: the photon pass runs beside the previous pass's gather and
-// takes 10/16 of the path-kernel grid, so the gather's kernels find free wave
-// slots instead of waiting for the persistent photon waves to drain.  On the
-// full-material workload (1M photons, 1024^2) a pass takes 3.95 ms with
-// 10/16, 4.03 with 9/16, 4.29 with 8/16, 3.94-4.47 with 11/16 and 4.04-4.58
-// with 12/16 (two steady states each), and 4.52 with the full grid, whose
-// photon waves starve the gather.
+// takes 8/16 of the path-kernel grid, so the gather's and the build's kernels
+// find free wave slots instead of waiting for the persistent photon waves to
+// drain.  Whole renders with 6/16, 8/16, 10/16, 12/16 and 14/16 (eye pass: 3/16
+// up to 12/16, then 2/16): full-material 1024^2 122.0, 118.9, 121.7, 120.5 and
+// 119.7 ms (32 passes), occluded light 51.0, 47.3, 50.5, 49.9 and 48.8 (16),
+// caustics with 4M photons 110.4, 100.3, 106.6, 105.6 and 110.0 (8), 256^2 10.3,
+// 10.0, 10.1, 10.1 and 10.2 (16).
 static void photon_pass(sppm_ctx* c, int step, const int* step_dev, hipStream_t st, bool beside_gather) {
     RenderBuffers& R = c->rb;
     TraceSpill sp = trace_spill(c);
-    if (beside_gather) sp.blocks = sp.blocks * 10 / 16 > 0 ? sp.blocks * 10 / 16 : 1;
+    if (beside_gather) sp.blocks = sp.blocks * 8 / 16 > 0 ? sp.blocks * 8 / 16 : 1;
     if (R.wave_bounces > 0) {
         int tb = R.wave_blocks;
-        if (beside_gather) tb = tb * 10 / 16 > 0 ? tb * 10 / 16 : 1;
+        if (beside_gather) tb = tb * 8 / 16 > 0 ? tb * 8 / 16 : 1;
         launch_photon_wave(c->scene.dev, R.slots, R.N, step, step_dev, R.wave, R.wave_bounces, R.wave_lanes, tb, sp,
                            c->guided ? &c->emit : nullptr, R.flags, photon_rays(R), st);
     } else {
