@@ -491,7 +491,19 @@ __global__ void k_guide_grad_reduce(const float* __restrict__ part, int nblocks,
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k > nparams) return;
     double s = 0.0;
-    for (int b = 0; b < nblocks; ++b) s += (double)part[(size_t)b * (nparams + 1) + k];
+    const size_t row = (size_t)nparams + 1;
+    int b = 0;
+    // 16 loads under way per thread (the sums keep their order): there are only
+    // about 1400 waves, and with one load after the other's addition the 93 MB of
+    // a 128 x 6 network's partials took 104 us
+    for (; b + 16 <= nblocks; b += 16) {
+        float v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = part[(b + j) * row + k];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) s += (double)v[j];
+    }
+    for (; b < nblocks; ++b) s += (double)part[b * row + k];
     if (k < nparams) {
         grad[k] = (float)(s / (double)GUIDE_GRAD_SCALE);
     } else {
