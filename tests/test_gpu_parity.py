@@ -203,13 +203,13 @@ def test_pass_parity_balanced_gather_full(full_scene_small):
 
 
 @pytest.mark.parametrize("w,h,N,r0", [(3, 3, 64, 0.3), (5, 7, 3000, 0.05), (33, 9, 40000, 0.004), (63, 65, 3000, 0.012),
-                                      (40, 31, 20000, 0.2)])
+                                      (40, 31, 20000, 0.2), (200, 170, 3000, 0.03)])
 def test_pass_parity_gather_edges(box_scene, w, h, N, r0):
     """The production gather's own neighbour pairs where its groups, rows and
     chunks are ragged: fewer hit points than a group, exactly one group, a
     partly filled last one, batches of a few photons over many rows, groups
-    that straddle the box (small radius, thousands of rows), and chunks of the
-    largest size."""
+    that straddle the box (small radius, thousands of rows), chunks of the
+    largest size, and more than 1024 groups (two per planning thread)."""
     run_parity(box_scene, scenes.pinhole_camera(w, h), 0.9, r0, N, 2, 4, f"gather edges {w}x{h}",
                record=sppm_amd.RECORD_PAIRS, max_pairs=40_000_000)
 
