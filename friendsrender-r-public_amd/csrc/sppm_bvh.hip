@@ -401,16 +401,17 @@ void free_bvh(BvhResult* r) {
 // slots between its two binary children).  The wide tree then follows the
 // decisions from the root, breadth first.  Node boxes are the binary nodes'
 // refitted boxes, so every triangle stays inside the boxes above it.
-// C_TRI = 0.15 with leaves of up to 8 triangles measured fastest on the
-// full-material scene (BVH8, three-axis SAH: 4.06 ms per pass against 4.13
-// at 0.1 and 4.27 at 0.07; with the longest-axis SAH 0.05 / 0.3 / 0.6 and
-// 4-triangle leaves were slower, and the photon pass took 2.88 ms against
-// 3.01 with the earlier greedy collapse, which opened the largest child
-// until a node had W).
+// C_TRI = 0.1 and C_LEAF = 1 with leaves of up to 8 triangles: the wave's lanes
+// share a leaf's triangles, so the leaf step itself costs more than they do.
+// Photon pass alone against 0.15 / 0.5: full-material scene 1.90 against 1.94 ms,
+// occluded light 1.13 against 1.17, caustics 5.94 against 5.96 (BVH8, three-axis
+// SAH; 0.1 / 0.5: 1.87, 1.18, 5.99; 0.25 / 0.5: 1.97, 1.20, 6.06; 0.4 / 0.5: 2.05,
+// 1.26, 6.35).  A greedy collapse, which opens the largest child until a node
+// has W, was 4 % slower than this program's first constants.
 namespace {
 constexpr float DP_C_NODE = 1.0f;
-constexpr float DP_C_TRI = 0.15f;
-constexpr float DP_C_LEAF = 0.5f;  // entering a leaf (pop, loop set-up): 4.03 ms per pass, 4.07 without
+constexpr float DP_C_TRI = 0.1f;
+constexpr float DP_C_LEAF = 1.0f;
 constexpr int DP_LEAF_MAX = 8;  // a leaf reference holds count - 1 in 3 bits, eight leaves' ends fit 7
 
 struct WideChild {
