@@ -24,6 +24,7 @@
 
 #include "../../include/sppm_amd.h"
 #include "sppm_guide.h"
+#include "sppm_guide_paths.h"
 #include "sppm_host_math.h"
 #include "sppm_kernels.h"
 #include "sppm_mtjump.h"
@@ -149,13 +150,7 @@ struct RenderBuffers {
     GroupBuffers groups{};
     int* pass_dev = nullptr;   // passes done (device copy of the pass counter, read by graph replays);
                                // [1], [2]: the same counted on the photon and eye streams of a replay
-    int* path_cell = nullptr;  // guided emission: emission cell per path, 2 x N (block = step parity)
-    float* path_ratio = nullptr;  // guided emission: q / p_plain per path, like path_cell
-    unsigned long long* pdep = nullptr;  // guided emission: deposited luminance per flattened photon (guide_fix)
-    // guided emission: this pass's photon offsets and stored count (N + 1),
-    // copied by the build for the gather's deposits and the training records,
-    // which run while the next pass stages its photons into off / nstored
-    int* doff = nullptr;
+    GuidePaths gpaths;         // guided emission
     uint32_t* flags = nullptr;
     Counters* ctr = nullptr;
     // closest-hit ray and tie counts, striped (STRIPES lines of RAY_STRIPE
@@ -173,6 +168,14 @@ struct RenderBuffers {
     int wave_bounces = 0;      // 0: the megakernel photon pass
     int wave_lanes = 0;        // lanes per ray of the trace kernel
     int wave_blocks = 0;       // trace kernel grid
+    int alloc_guide_paths() {
+        return guide_paths_alloc(gpaths, (size_t)N, (size_t)photon_cap,
+                                 [](void** p, size_t n) { return dalloc((char**)p, n); },
+                                 [](void* p) { (void)hipFree(p); });
+    }
+    void free_guide_paths() {
+        guide_paths_free(gpaths, [](void* p) { (void)hipFree(p); });
+    }
     void release() {
         dfree(pairs); dfree(npairs);
         dfree(wave.path.rng); dfree(wave.path.org); dfree(wave.path.dir); dfree(wave.path.ndir);
@@ -190,7 +193,7 @@ struct RenderBuffers {
         }
         hits = HitDev{};
         dfree(shared.rad); dfree(shared.cnt); dfree(shared.direct); dfree(counts); dfree(list_off); dfree(list_scan_tmp); dfree(lists);
-        dfree(words); dfree(cam_states); dfree(cam_phi); dfree(rstat); dfree(tiles); dfree(chunkp); dfree(chunk_off); dfree(partial); dfree(groups.keys); dfree(groups.vals); dfree(groups.tmp_k); dfree(groups.tmp_v); dfree(groups.hist); dfree(groups.nvalid); dfree(groups.chunkq); dfree(groups.stat); dfree(groups.spheres); dfree(pass_dev); dfree(path_cell); dfree(path_ratio); dfree(pdep); dfree(doff); dfree(flags); dfree(ctr); dfree(raystripes); dfree(image);
+        dfree(words); dfree(cam_states); dfree(cam_phi); dfree(rstat); dfree(tiles); dfree(chunkp); dfree(chunk_off); dfree(partial); dfree(groups.keys); dfree(groups.vals); dfree(groups.tmp_k); dfree(groups.tmp_v); dfree(groups.hist); dfree(groups.nvalid); dfree(groups.chunkq); dfree(groups.stat); dfree(groups.spheres); dfree(pass_dev); free_guide_paths(); dfree(flags); dfree(ctr); dfree(raystripes); dfree(image);
         lists_cap = 0;
         shape.clear();
         ready = false;
@@ -1097,16 +1100,14 @@ int sppm_begin(sppm_ctx* c) {
         R.shape = std::move(shape);
     }
     if (c->guided) {
-        if (!R.path_cell &&
-            ((rc = dalloc(&R.path_cell, 2 * (size_t)N)) || (rc = dalloc(&R.path_ratio, 2 * (size_t)N)) ||
-             (rc = dalloc(&R.pdep, R.photon_cap)) || (rc = dalloc(&R.doff, (size_t)N + 1)))) {
+        if ((rc = R.alloc_guide_paths())) {
             R.release();
             return rc;
         }
-        c->emit.path_cell = R.path_cell;
-        c->emit.path_ratio = c->gparams.target == SPPM_GUIDE_TARGET_RMS ? R.path_ratio : nullptr;
+        c->emit.path_cell = R.gpaths.cell;
+        c->emit.path_ratio = c->gparams.target == SPPM_GUIDE_TARGET_RMS ? R.gpaths.ratio : nullptr;
     } else {
-        dfree(R.path_cell); dfree(R.path_ratio); dfree(R.pdep); dfree(R.doff);
+        R.free_guide_paths();
     }
     HIPOK(hipMemsetAsync(R.counts, 0, sizeof(int) * (size_t)(np + 1), c->stream));
     launch_init_slots(R.slots, c->stream);
@@ -1255,8 +1256,8 @@ static void do_photons(sppm_ctx* c, int step, hipStream_t st, bool beside_gather
 static void do_guide(sppm_ctx* c, hipStream_t st, int step, const int* step_dev) {
     RenderBuffers& R = c->rb;
     const bool rms = c->gparams.target == SPPM_GUIDE_TARGET_RMS;
-    launch_guide_deposit(R.doff, R.doff + R.N, R.pdep, R.path_cell, rms ? R.path_ratio : nullptr, R.N, step, step_dev,
-                         c->guide.hpass, st);
+    launch_guide_deposit(R.gpaths.off, R.gpaths.off + R.N, R.gpaths.dep, R.gpaths.cell,
+                         rms ? R.gpaths.ratio : nullptr, R.N, step, step_dev, c->guide.hpass, st);
     const int every = c->gparams.train_interval > 1 ? c->gparams.train_interval : 1;
     if (!step_dev && step % every != 0) return;  // the deposits gather in the pass histogram until then
     guide_fold_hist(c->guide, c->gparams.history_decay, st);
@@ -1288,7 +1289,7 @@ static void do_publish(sppm_ctx* c, hipStream_t st) {
 // The rest of the build: grid, keys, sort and the cell-sorted records.
 static void do_build_grid(sppm_ctx* c, hipStream_t st) {
     RenderBuffers& R = c->rb;
-    if (c->guided) launch_copy_offsets(R.off, R.nstored, R.N, R.doff, st);
+    if (c->guided) launch_copy_offsets(R.off, R.nstored, R.N, R.gpaths.off, st);
     launch_build_grid(R.staged, R.nstored, R.ctr, R.gp, R.rstat, c->scene.bmin, c->scene.ext, R.cell_cap,
                       R.cell_start, R.cell_gaps, R.cell_ngap, R.psort, R.photon_cap, R.gpos, R.gflux, R.gdir, st);
 }
@@ -1356,11 +1357,11 @@ static int do_gather(sppm_ctx* c, hipStream_t st) {
                       R.ctr, R.flags, st);
         R.have_lists = true;
     } else {
-        if (c->guided) launch_deposit_clear(R.pdep, R.doff + R.N, st);
+        if (c->guided) launch_deposit_clear(R.gpaths.dep, R.gpaths.off + R.N, st);
         const PairRecord rec{R.pairs, R.npairs, R.pairs_cap};
         launch_gather_balanced(R.hits, R.shared, G, R.gp, R.np, c->scene.bmin, c->scene.ext, R.groups, alpha, R.tiles,
                                GATHER_CHUNK_CAP, R.chunkp, R.chunk_off, R.partial, R.counts,
-                               R.rstat, R.ctr, R.flags, c->guided ? R.pdep : nullptr, rec, st);
+                               R.rstat, R.ctr, R.flags, c->guided ? R.gpaths.dep : nullptr, rec, st);
         R.have_lists = R.pairs != nullptr;
     }
     if (c->scene.dev.ibl_tex >= 0 || c->params.eye_nee != SPPM_NEE_OFF) launch_direct_light(R.hits, R.shared, R.np, st);
@@ -1958,7 +1959,7 @@ static int prepare_multi(sppm_batch* b) {
         J.chunkp = R.chunkp;
         J.queue = R.groups.chunkq;
         J.partial = R.partial;
-        J.pdep = c->guided ? R.pdep : nullptr;
+        J.pdep = c->guided ? R.gpaths.dep : nullptr;
         J.rec = PairRecord{R.pairs, R.npairs, R.pairs_cap};
         gj.push_back(J);
         cj.push_back(CamJob{R.cam_states, R.cam_phi, R.cam_K, R.cam_L, R.words});
@@ -2038,7 +2039,7 @@ static int enqueue_multi(sppm_batch* b, hipStream_t st) {
     r = batch_branches(b, st, [&](int k, hipStream_t bs) {
         sppm_ctx* c = b->ctx[k];
         RenderBuffers& R = c->rb;
-        if (c->guided) launch_deposit_clear(R.pdep, R.doff + R.N, bs);
+        if (c->guided) launch_deposit_clear(R.gpaths.dep, R.gpaths.off + R.N, bs);
         const PairRecord rec{R.pairs, R.npairs, R.pairs_cap};
         (void)launch_gather_plan(R.hits, R.shared, grid_dev(c), R.gp, R.np, c->scene.bmin, c->scene.ext, R.groups,
                                  R.tiles, GATHER_CHUNK_CAP, R.chunkp, R.chunk_off, R.counts,
@@ -2785,6 +2786,9 @@ int sppm_guide_set(sppm_ctx* c, const sppm_guide_params* p) {
     GuideEmit E{};
     int rc = guide_light_frame(c, E);
     if (rc) return rc;
+    // whatever fails from here on leaves the context unguided: the emission
+    // tables and path buffers that a guided pass uses may be gone
+    c->guided = false;
     if (c->guide.theta && (c->guide.net.hidden != net.hidden || c->guide.net.layers != net.layers ||
                            c->guide.net.fp16 != net.fp16))
         guide_free(c->guide);
@@ -2822,19 +2826,13 @@ int sppm_guide_set(sppm_ctx* c, const sppm_guide_params* p) {
     E.w = p->mix_plain;
     E.prob = c->guide.eprob;
     E.cdf = c->guide.ecdf;
-    E.path_cell = c->rb.path_cell;
+    if (c->rb.ready && (rc = c->rb.alloc_guide_paths())) return rc;  // otherwise sppm_begin's
     c->emit = E;
     c->gparams = *p;
-    c->guided = true;
-    if (c->rb.ready && !c->rb.path_cell) {
-        RenderBuffers& R = c->rb;
-        if ((rc = dalloc(&R.path_cell, 2 * (size_t)R.N)) || (rc = dalloc(&R.path_ratio, 2 * (size_t)R.N)) ||
-            (rc = dalloc(&R.pdep, R.photon_cap)) || (rc = dalloc(&R.doff, (size_t)R.N + 1)))
-            return rc;
-        c->emit.path_cell = R.path_cell;
-    }
-    c->emit.path_ratio = p->target == SPPM_GUIDE_TARGET_RMS ? c->rb.path_ratio : nullptr;
+    c->emit.path_cell = c->rb.gpaths.cell;
+    c->emit.path_ratio = p->target == SPPM_GUIDE_TARGET_RMS ? c->rb.gpaths.ratio : nullptr;
     HIPOK(hipStreamSynchronize(c->stream));
+    c->guided = true;
     return SPPM_OK;
 }
 
@@ -2908,7 +2906,7 @@ int sppm_guide_path_cells(sppm_ctx* c, int32_t* cells) {
     // the emission of step s writes block s & 1; the last pass ran step pass + step_offset
     const long long step = (long long)c->pass + c->params.step_offset;
     HIPOK(hipStreamSynchronize(c->stream));
-    HIPOK(hipMemcpy(cells, c->rb.path_cell + (size_t)(step & 1) * (size_t)c->rb.N, sizeof(int) * (size_t)c->rb.N,
+    HIPOK(hipMemcpy(cells, c->rb.gpaths.cell + (size_t)(step & 1) * (size_t)c->rb.N, sizeof(int) * (size_t)c->rb.N,
                     hipMemcpyDeviceToHost));
     return SPPM_OK;
 }
