@@ -2903,6 +2903,8 @@ int sppm_guide_path_cells(sppm_ctx* c, int32_t* cells) {
     if (rc) return rc;
     if (!cells) return fail(SPPM_E_ARG, "NULL output");
     if (c->pass < 1) return fail(SPPM_E_STATE, "no pass rendered since sppm_begin");
+    // guided emission may have been turned off since, and the render begun without it
+    if (!c->rb.gpaths.cell) return fail(SPPM_E_STATE, "the render was begun without guided emission");
     // the emission of step s writes block s & 1; the last pass ran step pass + step_offset
     const long long step = (long long)c->pass + c->params.step_offset;
     HIPOK(hipStreamSynchronize(c->stream));

@@ -217,3 +217,19 @@ def test_guided_lowers_per_pass_variance():
     print("variance gain %.2f; image total plain %.4g guided %.4g" % (gain, tp, tg), flush=True)
     assert abs(tg - tp) < 0.03 * tp
     assert gain > 1.15
+
+
+def test_path_cells_refused_without_guided_buffers(box_scene):
+    """The path cells of a render begun after guided emission was turned off:
+    there are none, which is an error and no read."""
+    r = sppm_amd.Renderer(box_scene, scenes.pinhole_camera(16, 16), 0.9, 0.05, 1000, bvh_width=4)
+    r.guide_set(True, learning_rate=1e-3, train_steps=1)
+    r.begin()
+    r.pass_()
+    assert len(r.guide_path_cells()) == 1000
+    r.guide_set(False)
+    r.begin()
+    r.pass_()
+    with pytest.raises(sppm_amd.SppmError, match="without guided emission"):
+        r.guide_path_cells()
+    r.close()
