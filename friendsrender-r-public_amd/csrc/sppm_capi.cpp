@@ -1186,22 +1186,29 @@ static TraceSpill trace_spill(const sppm_ctx* c) {
     if (c->tuned_blocks > 0 && c->tuned_blocks < sp.blocks) sp.blocks = c->tuned_blocks;
     return sp;
 }
-// the eye pass's own spill area: in a full pass it runs beside the photon pass
-// beside: in a full pass it takes 3/16 of the path-kernel grid.  Its persistent
-// waves would otherwise fill every wave slot that the gather leaves free, and
-// the build's short kernels after it wait for them (a sort pass took 1.5 ms):
-// 4M photons at 1024^2 (caustics, 8 passes) 124.5 ms with 5/16 against 135.5 with
-// the whole grid.  With 8/16 for the photons (photon_pass) 3/16 against 5/16
-// and 10/16: occluded light at 1024^2 47.3 against 52.3 ms (16 passes), 256^2
-// 10.0 against 10.4, full-material 1024^2 118.9 against 120.5 (32 passes).
-// With next-event estimation the eye pass is as long as the photon pass and
-// takes 5/16: 400x300 pixels 6.45 ms, 7.40 with 3/16, 6.54 with 4/16, 6.56 with
-// 7/16 and 6.71 with the whole grid (8 passes).
+// The eye pass's own spill area: in a full pass it runs beside the photon pass.
+// beside: it then takes a share of the path-kernel grid.  Its persistent waves
+// would otherwise fill the wave slots that the photon pass (photon_pass) and
+// the gather leave free, and the build's short kernels after it wait for them.
+// The photon pass takes 8/16, so the eye pass takes as many sixteenths as lets
+// the two last equally long, and at least 3: its work in photon paths (2.3 rays
+// of a path spread all over the scene) is 0.9 rays a pixel (1.1 traced, from one
+// point), 1.7 with next-event estimation, 3 where paths go on to an environment
+// (3 to 4 traced).  8 passes in ms with 3/16, 5/16 and this share: 1024^2 with an
+// environment and 300k photons 41.0, 29.5, 20.1; 1024^2 and 100k photons 14.4,
+// 12.4, 11.3; 1024^2 with next-event estimation, 200k and 1M photons 22.8, 18.8,
+// 15.5 and 29.6, 26.4, 23.9.  Where the photon pass is the longer one the share
+// matters little: 32 passes of full-material 1024^2 (1M photons) 117.7 with 3/16,
+// 115.3 with the whole grid; 4M photons (caustics, 8 passes) 104.8 with 2/16,
+// 100.7 with 3/16, 101.3 with the whole grid; 16 of 512^2 (250k photons) 23.0
+// with 3/16, 23.5 with 12/16.
 static TraceSpill trace_spill_eye(const sppm_ctx* c, bool beside) {
     TraceSpill sp = c->scene.trace_spill_eye();
     if (beside) {
-        const int share = c->params.eye_nee != SPPM_NEE_OFF ? 5 : 3;
-        sp.blocks = sp.blocks * share / 16 > 0 ? sp.blocks * share / 16 : 1;
+        const double per_pixel = c->scene.dev.ibl_tex >= 0 ? 3.0 : c->params.eye_nee != SPPM_NEE_OFF ? 1.7 : 0.9;
+        const double eye = per_pixel * c->rb.np, photons = 2.3 * c->rb.N;
+        const int share = (int)std::min(16.0, std::max(3.0, std::round(8.0 * eye / photons)));
+        sp.blocks = std::max(1, sp.blocks * share / 16);
     }
     if (c->tuned_blocks > 0 && c->tuned_blocks < sp.blocks) sp.blocks = c->tuned_blocks;
     return sp;

@@ -21,6 +21,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "sppm_guide.h"
 #include "sppm_kernels.h"
 #include "sppm_pass.h"
@@ -1847,8 +1849,11 @@ static void launch_eye_t(const SceneDev& S, const CamDev& C, const HitDev& H, in
                          const TraceSpill& sp, const uint32_t* words, uint32_t* flags, unsigned long long* rays,
                          int* queue, int keep, hipStream_t st) {
     hipLaunchKernelGGL(k_zero_i32, dim3(STRIPE_INTS / 256), dim3(256), 0, st, queue, STRIPE_INTS);
-    dim3 g(sp.blocks), b(PATH_BLOCK);
     const int claim = wave_share((long long)C.W * C.H);
+    // no more waves than claims (of each stripe): the others would only take
+    // slots from the photon pass and the short kernels beside
+    const int per = (C.W * C.H + STRIPES - 1) / STRIPES;
+    dim3 g(std::min(sp.blocks, STRIPES * ((per + claim - 1) / claim))), b(PATH_BLOCK);
     if (S.width == 2)
         hipLaunchKernelGGL((k_eye<2, NEE>), g, b, 0, st, S, C, H, step, step_dev, sp.cap, sp.buf, words, flags, keep,
                            rays, queue, claim);
