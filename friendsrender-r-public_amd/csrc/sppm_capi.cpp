@@ -193,7 +193,7 @@ struct RenderBuffers {
         }
         hits = HitDev{};
         dfree(shared.rad); dfree(shared.cnt); dfree(shared.direct); dfree(counts); dfree(list_off); dfree(list_scan_tmp); dfree(lists);
-        dfree(words); dfree(cam_states); dfree(cam_phi); dfree(rstat); dfree(tiles); dfree(chunkp); dfree(chunk_off); dfree(partial); dfree(groups.keys); dfree(groups.vals); dfree(groups.tmp_k); dfree(groups.tmp_v); dfree(groups.hist); dfree(groups.nvalid); dfree(groups.chunkq); dfree(groups.stat); dfree(groups.spheres); dfree(pass_dev); free_guide_paths(); dfree(flags); dfree(ctr); dfree(raystripes); dfree(image);
+        dfree(words); dfree(cam_states); dfree(cam_phi); dfree(rstat); dfree(tiles); dfree(chunkp); dfree(chunk_off); dfree(partial); dfree(groups.keys); dfree(groups.vals); dfree(groups.tmp_k); dfree(groups.tmp_v); dfree(groups.hist); dfree(groups.nvalid); dfree(groups.chunkq); dfree(groups.stat); dfree(groups.cand); dfree(groups.spheres); dfree(pass_dev); free_guide_paths(); dfree(flags); dfree(ctr); dfree(raystripes); dfree(image);
         lists_cap = 0;
         shape.clear();
         ready = false;
@@ -1044,7 +1044,8 @@ int sppm_begin(sppm_ctx* c) {
             (rc = dalloc(&R.raystripes, (size_t)STRIPES * RAY_STRIPE)) ||
             (rc = dalloc((char**)&R.tiles, gather_tile_bytes() * (size_t)ntile_max)) ||
             (rc = dalloc(&R.chunkp, 1)) ||
-            (rc = dalloc(&R.chunk_off, ntile_max + 1)) ||
+            (rc = dalloc(&R.chunk_off, gather_plan_entries(gather_group_count(np)))) ||
+            (rc = dalloc(&R.groups.cand, gather_plan_entries(gather_group_count(np)))) ||
             (rc = dalloc(&R.partial, (size_t)64 * (GATHER_CHUNK_CAP + ntile_max))) ||
             (rc = dalloc(&R.groups.keys, np)) || (rc = dalloc(&R.groups.vals, np)) || (rc = dalloc(&R.groups.tmp_k, np)) ||
             (rc = dalloc(&R.groups.tmp_v, np)) || (rc = dalloc(&R.groups.hist, radix_hist_entries(np))) ||
@@ -1964,6 +1965,7 @@ static int prepare_multi(sppm_batch* b) {
         J.order = gather_order(R.groups, R.np);
         J.nvalid = R.groups.nvalid;
         J.tiles = R.tiles;
+        J.cand = R.groups.cand;
         J.spheres = R.groups.spheres;
         J.ntiles = gather_group_count(R.np);
         J.chunk_off = R.chunk_off;

@@ -129,6 +129,7 @@ struct GroupBuffers {
     int* nvalid;  // valid hit points
     int* chunkq;  // striped chunk counters of the gather (STRIPE_INTS)
     unsigned long long* stat;  // 3 per group: radius sum, active hit points, neighbours
+    int* cand;    // candidate photons of every group (gather_plan_entries(groups))
     float4* spheres;  // query sphere of every grouped hit point (gather_sphere_entries(np))
 };
 // Neighbour pairs (hit point, flattened photon index) that the production
@@ -159,6 +160,7 @@ void launch_gather_finish(const HitDev& H, const SharedDev& SH, int np, const ui
                           float alpha, const int* chunk_off, const float4* partial, int* counts,
                           unsigned long long* rstat, Counters* ctr, uint32_t* flags, hipStream_t st);
 int gather_group_count(int np);
+size_t gather_plan_entries(int ngroups);  // of cand and chunk_off: with the end, to a multiple of four
 size_t gather_sphere_entries(int np);
 int gather_tile_count(int W, int Hh);
 size_t gather_tile_bytes();
@@ -202,6 +204,7 @@ struct GatherJob {
     const uint32_t* order;
     const int* nvalid;
     const TileRange* tiles;
+    const int* cand;
     const float4* spheres;
     int ntiles;
     const int* chunk_off;

@@ -1066,7 +1066,7 @@ __global__ void __launch_bounds__(64) k_gather(HitDev H, SharedDev SH, GridDev G
 //   k_gather_finish  per tile: partial sums in chunk order + the update
 // ---------------------------------------------------------------------------
 struct TileRange {
-    int x0, x1, y0, y1, z0, z1, rowlen_pad, cand;
+    int y0, y1, z0, z1;
 };
 
 // Hit-point groups of the balanced gather: the valid hit points sorted by the
@@ -1226,7 +1226,8 @@ constexpr float SPHERE_MARGIN = 0x1p-18f;
 // Per group: its union cell box, its candidate count and its query spheres.
 __global__ void __launch_bounds__(64) k_gather_plan(HitDev H, SharedDev SH, GridDev G, const GridParams* __restrict__ gp,
                                                     const uint32_t* __restrict__ order, const int* __restrict__ nvalidp,
-                                                    TileRange* __restrict__ tiles, float4* __restrict__ spheres) {
+                                                    TileRange* __restrict__ tiles, int* __restrict__ cand,
+                                                    float4* __restrict__ spheres) {
     const int lane = threadIdx.x;
     const int p = lane < GATHER_GROUP ? group_pixel(order, *nvalidp, blockIdx.x * GATHER_GROUP + lane) : -1;
     const GridParams g = *gp;
@@ -1253,21 +1254,21 @@ __global__ void __launch_bounds__(64) k_gather_plan(HitDev H, SharedDev SH, Grid
         if (lane == 0) sp[2 * GATHER_GROUP] = make_float4(o.x, o.y, o.z, far < 1e30f && far < 512.0f * rmin ? far : -1.0f);
     }
     TileRange T;
-    T.x0 = -wave_max_i(active ? -r[0] : -0x7fffffff); T.x1 = wave_max_i(active ? r[1] : -1);
     T.y0 = -wave_max_i(active ? -r[2] : -0x7fffffff); T.y1 = wave_max_i(active ? r[3] : -1);
     T.z0 = -wave_max_i(active ? -r[4] : -0x7fffffff); T.z1 = wave_max_i(active ? r[5] : -1);
-    int cand = 0;
+    int n = 0;
     if (__ballot(active)) {
         const int ny = __builtin_amdgcn_readfirstlane(T.y1 - T.y0 + 1);
         const int nrows = __builtin_amdgcn_readfirstlane(ny * (T.z1 - T.z0 + 1));
-        for (int k0 = 0; k0 < nrows; k0 += 64) cand += group_rows(T, ny, nrows, k0, r, active, g, G.cell_start).len;
+        for (int k0 = 0; k0 < nrows; k0 += 64) n += group_rows(T, ny, nrows, k0, r, active, g, G.cell_start).len;
     } else {
-        T.x0 = 0; T.x1 = -1; T.y0 = 0; T.y1 = -1; T.z0 = 0; T.z1 = -1;
+        T.y0 = 0; T.y1 = -1; T.z0 = 0; T.z1 = -1;
     }
-    cand = wave_sum_i(cand);
-    T.rowlen_pad = 0;
-    T.cand = cand;
-    if (lane == 0) tiles[blockIdx.x] = T;
+    n = wave_sum_i(n);
+    if (lane == 0) {
+        tiles[blockIdx.x] = T;
+        cand[blockIdx.x] = n;
+    }
 }
 
 // Candidates per chunk, a multiple of 64: about GATHER_CHUNKS_PER_WAVE chunks
@@ -1278,51 +1279,93 @@ __global__ void __launch_bounds__(64) k_gather_plan(HitDev H, SharedDev SH, Grid
 // hundred waves.
 constexpr int GATHER_CHUNKS_PER_WAVE = 2;
 // One workgroup makes the chunk size, every group's chunk count and their
-// offsets (chunk_off[ntiles]: all chunks): six short launches before, whose
-// own 4 to 5 us each were a tenth of a small render's pass.
+// offsets (chunk_off[ntiles]: all chunks).  It is bound by the latency of its
+// loads and, beyond some ten thousand groups, by its one CU: neighbouring lanes
+// read neighbouring counts, four at a time, and the offsets are scanned 4096
+// groups a step.  Alone 5.0, 13 and 38 us at 256^2, 1024^2 and 2048^2; with
+// each thread on its own run of 32-byte records, three times over, 6.6, 79 and
+// 355; as six launches (a sum by one workgroup, the counts, a scan) 27, 64 and
+// 160.
+// cand and chunk_off hold gather_plan_entries(ntiles) ints; cand past ntiles is
+// not read as a count.
 constexpr int CHUNK_THREADS = 1024;
-__global__ void __launch_bounds__(CHUNK_THREADS) k_chunks(const TileRange* __restrict__ tiles, int ntiles, int cap,
+constexpr int CHUNK_STEP = 4 * CHUNK_THREADS;  // groups a step
+__device__ __forceinline__ int4 cand_load(const int* __restrict__ cand, int t, int ntiles) {
+    if (t > ntiles) return make_int4(0, 0, 0, 0);
+    int4 v = *reinterpret_cast<const int4*>(cand + t);
+    v.x = t < ntiles ? v.x : 0;
+    v.y = t + 1 < ntiles ? v.y : 0;
+    v.z = t + 2 < ntiles ? v.z : 0;
+    v.w = t + 3 < ntiles ? v.w : 0;
+    return v;
+}
+__global__ void __launch_bounds__(CHUNK_THREADS) k_chunks(const int* __restrict__ cand, int ntiles, int cap,
                                                           int* __restrict__ chunk, int* __restrict__ chunk_off,
                                                           Counters* __restrict__ ctr) {
-    __shared__ unsigned long long part[CHUNK_THREADS / 64];
-    __shared__ int wsum[CHUNK_THREADS / 64], sh_chunk;
+    constexpr int WAVES = CHUNK_THREADS / 64;
+    __shared__ unsigned long long part[WAVES];
+    __shared__ int wsum[2][WAVES];
+    __shared__ unsigned sh_chunk;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int per = (ntiles + CHUNK_THREADS - 1) / CHUNK_THREADS;
-    const int t0 = min((int)threadIdx.x * per, ntiles), t1 = min(t0 + per, ntiles);
+    const int mine = 4 * (int)threadIdx.x;
     unsigned long long s = 0;
-    for (int t = t0; t < t1; ++t) s += (unsigned long long)tiles[t].cand;
+#pragma unroll 4
+    for (int t = mine; t < ntiles; t += CHUNK_STEP) {
+        const int4 v = cand_load(cand, t, ntiles);
+        s += (unsigned long long)v.x + (unsigned long long)v.y + (unsigned long long)v.z + (unsigned long long)v.w;
+    }
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
     if (lane == 0) part[wave] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
         unsigned long long tot = 0;
-        for (int w = 0; w < CHUNK_THREADS / 64; ++w) tot += part[w];
+        for (int w = 0; w < WAVES; ++w) tot += part[w];
         unsigned long long c = (tot + (unsigned long long)cap - 1) / (unsigned long long)cap;
         unsigned long long lo = tot / (unsigned long long)(GATHER_WAVES * GATHER_CHUNKS_PER_WAVE);
         lo = lo < 128 ? 128 : lo > 1024 ? 1024 : lo;
         if (c < lo) c = lo;
         c = (c + 63) & ~63ull;
-        *chunk = sh_chunk = (int)c;
+        sh_chunk = (unsigned)c;
+        *chunk = (int)c;
         ctr->candidates += tot;
     }
     __syncthreads();
-    const int c = sh_chunk;
-    int n = 0;
-    for (int t = t0; t < t1; ++t) n += (tiles[t].cand + c - 1) / c;
-    int incl = n;
-    for (int off = 1; off < 64; off <<= 1) {
-        const int v = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += v;
+    const unsigned c = sh_chunk, inv = 0xffffffffu / c;
+    // ceil(v / c): the product with the rounded-down reciprocal is at most one short
+    const auto chunks = [c, inv](int v) {
+        const unsigned x = (unsigned)v + c - 1u;
+        const unsigned q = __umulhi(x, inv);
+        return (int)(q + (x - q * c >= c ? 1u : 0u));
+    };
+    int done = 0;  // chunks of the steps before
+    int4 next = cand_load(cand, mine, ntiles);
+    // up to and with ntiles, the entry of all chunks
+    for (int base = 0, k = 0; base <= ntiles; base += CHUNK_STEP, k ^= 1) {
+        const int t = base + mine;
+        const int4 v = next;
+        next = cand_load(cand, t + CHUNK_STEP, ntiles);
+        int4 o;  // exclusive sums of the thread's four
+        o.x = 0;
+        o.y = chunks(v.x);
+        o.z = o.y + chunks(v.y);
+        o.w = o.z + chunks(v.z);
+        const int n = o.w + chunks(v.w);
+        int incl = n;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int u = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += u;
+        }
+        if (lane == 63) wsum[k][wave] = incl;
+        __syncthreads();  // the next step writes the other half of wsum
+        int run = done + incl - n;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const int u = wsum[k][w];
+            run += w < wave ? u : 0;
+            done += u;
+        }
+        if (t <= ntiles) *reinterpret_cast<int4*>(chunk_off + t) = make_int4(run + o.x, run + o.y, run + o.z, run + o.w);
     }
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    int run = incl - n;
-    for (int w = 0; w < wave; ++w) run += wsum[w];
-    for (int t = t0; t < t1; ++t) {
-        chunk_off[t] = run;
-        run += (tiles[t].cand + c - 1) / c;
-    }
-    if (threadIdx.x == CHUNK_THREADS - 1) chunk_off[ntiles] = run;
 }
 
 // Transposes the 32 x 32 bit matrix that each half of the wave holds, a row
@@ -1375,8 +1418,8 @@ __device__ __forceinline__ uint32_t transpose32(uint32_t x, int lane) {
 __device__ __forceinline__ void gather_chunks(HitDev H, SharedDev SH, GridDev G,
                                               const GridParams* __restrict__ gp, const uint32_t* __restrict__ order,
                                               const int* __restrict__ nvalidp, const TileRange* __restrict__ tiles,
-                                              const float4* __restrict__ spheres, int ntiles,
-                                              const int* __restrict__ chunk_off, const int* __restrict__ chunkp,
+                                              const int* __restrict__ cand, const float4* __restrict__ spheres,
+                                              int ntiles, const int* __restrict__ chunk_off, const int* __restrict__ chunkp,
                                               int* __restrict__ queue, float4* __restrict__ partial,
                                               unsigned long long* __restrict__ pdep, PairRecord rec) {
     // LDS of the loop (one wave per block; each kernel that inlines this
@@ -1422,8 +1465,8 @@ __device__ __forceinline__ void gather_chunks(HitDev H, SharedDev SH, GridDev G,
         // the pixel weight multiplies the sum, unless it is not finite (then
         // every term, as W * BRDF * Flux / PDF gives NaN for a zero factor)
         const bool wfin = isfinite(L.wgt.x) && isfinite(L.wgt.y) && isfinite(L.wgt.z);
-        const int first = (ch - chunk_off[t]) * CH;
-        const int last = T.cand - first > CH ? first + CH : T.cand;
+        const int first = (ch - chunk_off[t]) * CH, all = cand[t];
+        const int last = all - first > CH ? first + CH : all;
         const int ny = T.y1 - T.y0 + 1, nrows = ny * (T.z1 - T.z0 + 1);
         int acc = 0;  // candidates before the current block of rows
         for (int k0 = 0; k0 < nrows && acc < last; k0 += 64) {
@@ -1566,11 +1609,12 @@ __global__ void __launch_bounds__(64) k_gather_chunks(HitDev H, SharedDev SH, Gr
                                                       const GridParams* __restrict__ gp,
                                                       const uint32_t* __restrict__ order, const int* __restrict__ nvalidp,
                                                       const TileRange* __restrict__ tiles,
+                                                      const int* __restrict__ cand,
                                                       const float4* __restrict__ spheres, int ntiles,
                                                       const int* __restrict__ chunk_off, const int* __restrict__ chunkp,
                                                       int* __restrict__ queue, float4* __restrict__ partial,
                                                       unsigned long long* __restrict__ pdep, PairRecord rec) {
-    gather_chunks(H, SH, G, gp, order, nvalidp, tiles, spheres, ntiles, chunk_off, chunkp, queue, partial, pdep, rec);
+    gather_chunks(H, SH, G, gp, order, nvalidp, tiles, cand, spheres, ntiles, chunk_off, chunkp, queue, partial, pdep, rec);
 }
 
 // The gather chunks of every scene of a batch (see k_photon_multi).
@@ -1581,8 +1625,8 @@ __global__ void __launch_bounds__(64, GATHER_WAVES_PER_SIMD) k_gather_chunks_mul
         const int s = __builtin_amdgcn_readfirstlane(home + k < njobs ? home + k : home + k - njobs);
         const GatherJob& J = jobs[s];
         if (scene_done(J.queue)) continue;
-        gather_chunks(J.H, J.SH, J.G, J.gp, J.order, J.nvalid, J.tiles, J.spheres, J.ntiles, J.chunk_off, J.chunkp, J.queue,
-                      J.partial, J.pdep, J.rec);
+        gather_chunks(J.H, J.SH, J.G, J.gp, J.order, J.nvalid, J.tiles, J.cand, J.spheres, J.ntiles, J.chunk_off, J.chunkp,
+                      J.queue, J.partial, J.pdep, J.rec);
         scene_mark_done(J.queue);
     }
 }
@@ -1951,8 +1995,9 @@ const uint32_t* launch_gather_plan(const HitDev& H, const SharedDev& SH, const G
     const SortResult sr = radix_sort_pairs(gb.keys, gb.vals, gb.tmp_k, gb.tmp_v, gb.hist, np, 31, st);
     hipLaunchKernelGGL(k_count_valid, dim3(1), dim3(64), 0, st, sr.keys, np, gb.nvalid);
     const uint32_t* order = sr.vals;  // == gather_order(gb, np)
-    hipLaunchKernelGGL(k_gather_plan, dim3(ntiles), dim3(64), 0, st, H, SH, G, gp, order, gb.nvalid, tiles, gb.spheres);
-    hipLaunchKernelGGL(k_chunks, dim3(1), dim3(CHUNK_THREADS), 0, st, tiles, ntiles, cap, chunkp, chunk_off, ctr);
+    hipLaunchKernelGGL(k_gather_plan, dim3(ntiles), dim3(64), 0, st, H, SH, G, gp, order, gb.nvalid, tiles, gb.cand,
+                       gb.spheres);
+    hipLaunchKernelGGL(k_chunks, dim3(1), dim3(CHUNK_THREADS), 0, st, gb.cand, ntiles, cap, chunkp, chunk_off, ctr);
     if (rec.pairs) launch_set_u64x2(rec.count, 0ull, 0ull, st);
     return order;
 }
@@ -1961,7 +2006,7 @@ void launch_gather_run(const HitDev& H, const SharedDev& SH, const GridDev& G, c
                        const int* chunk_off, float4* partial, unsigned long long* pdep, const PairRecord& rec,
                        hipStream_t st) {
     hipLaunchKernelGGL(k_gather_chunks, dim3(GATHER_WAVES), dim3(64), 0, st, H, SH, G, gp, order, gb.nvalid, tiles,
-                       gb.spheres, gather_group_count(np), chunk_off, chunkp, gb.chunkq, partial, pdep, rec);
+                       gb.cand, gb.spheres, gather_group_count(np), chunk_off, chunkp, gb.chunkq, partial, pdep, rec);
 }
 void launch_gather_finish(const HitDev& H, const SharedDev& SH, int np, const uint32_t* order, const GroupBuffers& gb,
                           float alpha, const int* chunk_off, const float4* partial, int* counts,
@@ -2022,6 +2067,7 @@ const uint32_t* gather_order(const GroupBuffers& gb, int np) {
 }
 int gather_tile_count(int W, int Hh) { return ((W + 7) >> 3) * ((Hh + 7) >> 3); }
 int gather_group_count(int np) { return (np + GATHER_GROUP - 1) / GATHER_GROUP; }
+size_t gather_plan_entries(int ngroups) { return ((size_t)ngroups + 4) / 4 * 4; }
 size_t gather_sphere_entries(int np) { return (size_t)gather_group_count(np) * SPHERES; }
 size_t gather_tile_bytes() { return sizeof(TileRange); }
 

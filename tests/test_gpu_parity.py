@@ -214,6 +214,29 @@ def test_pass_parity_gather_edges(box_scene, w, h, N, r0):
                record=sppm_amd.RECORD_PAIRS, max_pairs=40_000_000)
 
 
+@pytest.mark.parametrize("w,h", [(4, 5), (16, 8), (546, 240), (512, 256), (396, 331), (724, 363)])
+def test_gather_chunk_offsets_by_group_count(w, h, box_scene):
+    """Chunk offsets for 1, 4, 4095, 4096, 4097 and 8213 hit-point groups (they
+    are scanned four at a time, 4096 a step): the neighbour counts of every hit
+    point against the recording gather's, which has no chunks."""
+    say(f"gather chunk offsets: {w}x{h}")
+    cam = scenes.pinhole_camera(w, h)
+    rs = [sppm_amd.Renderer(box_scene, cam, 0.9, 0.02, 6000, bvh_width=8, record=rec) for rec in (False, True)]
+    for _ in range(2):
+        for r in rs:
+            r.pass_()
+        a, b = (r.read_counts() for r in rs)
+        assert a.sum() > 0
+        np.testing.assert_array_equal(a, b)
+    a, b = (r.counters() for r in rs)
+    assert (a["hit_points"], a["neighbours"]) == (b["hit_points"], b["neighbours"])
+    a, b = (r.read_shared() for r in rs)
+    np.testing.assert_array_equal(a["radius"], b["radius"])
+    np.testing.assert_allclose(a["radiance"], b["radiance"], rtol=1e-4, atol=1e-4 * float(b["radiance"].max()))
+    for r in rs:
+        r.close()
+
+
 @pytest.mark.parametrize("w,h", [(3, 3), (7, 5), (19, 4), (37, 7), (119, 61)])
 def test_camera_words_sizes(w, h, box_scene):
     """Three passes' camera words at sizes around the generator's own (227 words
