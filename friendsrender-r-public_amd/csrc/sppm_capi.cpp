@@ -143,7 +143,6 @@ struct RenderBuffers {
     long long cam_L = 0;
     unsigned long long* rstat = nullptr;  // (radius sum in 2^-32 units, hit points) of the last gather
     TileRange* tiles = nullptr;
-    int ntiles = 0;
     int* chunkp = nullptr;
     int* chunk_off = nullptr;
     float4* partial = nullptr;
@@ -1023,8 +1022,7 @@ int sppm_begin(sppm_ctx* c) {
     if (!keep) {
         R.release();
         R.N = N; R.W = W; R.H = Hh; R.np = np;
-        // tiles of the recording gather (8x8 pixels) or hit-point groups of the production gather
-        const int ntile_max = std::max(gather_tile_count(W, Hh), gather_group_count(np));
+        const int ngroups = gather_group_count(np);
         R.slots.npaths = N;
         if ((rc = dalloc(&R.slots.pos, NS)) || (rc = dalloc(&R.slots.flux, NS)) || (rc = dalloc(&R.slots.dir, NS)) ||
             (rc = dalloc(&R.slots.valid, NS)) || (rc = dalloc(&R.slots.count, N)) || (rc = dalloc(&R.off, N)) ||
@@ -1042,14 +1040,14 @@ int sppm_begin(sppm_ctx* c) {
             (rc = dalloc(&R.words, 2 * 6 * (size_t)np)) || (rc = dalloc(&R.cam_phi, MT_WORDS)) ||
             (rc = dalloc(&R.rstat, 2)) || (rc = dalloc(&R.flags, 1)) || (rc = dalloc(&R.ctr, 1)) ||
             (rc = dalloc(&R.raystripes, (size_t)STRIPES * RAY_STRIPE)) ||
-            (rc = dalloc((char**)&R.tiles, gather_tile_bytes() * (size_t)ntile_max)) ||
+            (rc = dalloc((char**)&R.tiles, gather_tile_bytes() * (size_t)ngroups)) ||
             (rc = dalloc(&R.chunkp, 1)) ||
-            (rc = dalloc(&R.chunk_off, gather_plan_entries(gather_group_count(np)))) ||
-            (rc = dalloc(&R.groups.cand, gather_plan_entries(gather_group_count(np)))) ||
-            (rc = dalloc(&R.partial, (size_t)64 * (GATHER_CHUNK_CAP + ntile_max))) ||
+            (rc = dalloc(&R.chunk_off, gather_plan_entries(ngroups))) ||
+            (rc = dalloc(&R.groups.cand, gather_plan_entries(ngroups))) ||
+            (rc = dalloc(&R.partial, gather_partial_entries(ngroups))) ||
             (rc = dalloc(&R.groups.keys, np)) || (rc = dalloc(&R.groups.vals, np)) || (rc = dalloc(&R.groups.tmp_k, np)) ||
             (rc = dalloc(&R.groups.tmp_v, np)) || (rc = dalloc(&R.groups.hist, radix_hist_entries(np))) ||
-            (rc = dalloc(&R.groups.nvalid, 1)) || (rc = dalloc(&R.groups.chunkq, STRIPE_INTS)) || (rc = dalloc(&R.groups.stat, 3 * (size_t)gather_group_count(np))) ||
+            (rc = dalloc(&R.groups.nvalid, 1)) || (rc = dalloc(&R.groups.chunkq, STRIPE_INTS)) || (rc = dalloc(&R.groups.stat, 3 * (size_t)ngroups)) ||
             (rc = dalloc(&R.groups.spheres, gather_sphere_entries(np))) ||
             (rc = dalloc(&R.pass_dev, 3)) ||
             (rc = dalloc(&R.image, np))) {
@@ -1127,7 +1125,6 @@ int sppm_begin(sppm_ctx* c) {
             return rc;
         }
     }
-    R.ntiles = gather_tile_count(W, Hh);
     launch_set_u64x2(R.rstat, (unsigned long long)((double)c->params.first_radius * 4294967296.0), 1ull, c->stream);
     launch_set_u32(R.flags, 0u, c->stream);
     launch_set_u32(reinterpret_cast<uint32_t*>(R.nstored), 0u, c->stream);

@@ -160,9 +160,9 @@ void launch_gather_finish(const HitDev& H, const SharedDev& SH, int np, const ui
                           float alpha, const int* chunk_off, const float4* partial, int* counts,
                           unsigned long long* rstat, Counters* ctr, uint32_t* flags, hipStream_t st);
 int gather_group_count(int np);
+size_t gather_partial_entries(int ngroups);
 size_t gather_plan_entries(int ngroups);  // of cand and chunk_off: with the end, to a multiple of four
 size_t gather_sphere_entries(int np);
-int gather_tile_count(int W, int Hh);
 size_t gather_tile_bytes();
 void launch_set_u64x2(unsigned long long* p, unsigned long long a, unsigned long long b, hipStream_t st);
 

@@ -2065,8 +2065,10 @@ int gather_wave_count() { return GATHER_WAVES; }
 const uint32_t* gather_order(const GroupBuffers& gb, int np) {
     return radix_sort_result(gb.keys, gb.vals, gb.tmp_k, gb.tmp_v, np, 31).vals;
 }
-int gather_tile_count(int W, int Hh) { return ((W + 7) >> 3) * ((Hh + 7) >> 3); }
 int gather_group_count(int np) { return (np + GATHER_GROUP - 1) / GATHER_GROUP; }
+// a slot per hit point of a group for every chunk: at most the budget's, and
+// one more per group from rounding up
+size_t gather_partial_entries(int ngroups) { return (size_t)GATHER_GROUP * (GATHER_CHUNK_CAP + (size_t)ngroups); }
 size_t gather_plan_entries(int ngroups) { return ((size_t)ngroups + 4) / 4 * 4; }
 size_t gather_sphere_entries(int np) { return (size_t)gather_group_count(np) * SPHERES; }
 size_t gather_tile_bytes() { return sizeof(TileRange); }
