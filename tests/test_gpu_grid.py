@@ -57,12 +57,44 @@ def test_grid_layout_full_workload():
     r.close()
 
 
-@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 4194304, 4194305])
-def test_photon_offsets_scan_sizes(n, box_scene):
-    """The stored photons of path counts around a scan tile (2048) and around
-    the tile count where the scan of the tile sums becomes a launch of its own."""
-    r = sppm_amd.Renderer(box_scene, scenes.pinhole_camera(8, 8), 0.9, 0.015, n, bvh_width=8)
-    r.photons(1)
-    stored = r.build()
-    assert stored == int(r.read_path_counts().astype(np.int64).sum())
+SCAN_TILE = 2048
+
+
+@pytest.fixture(scope="module")
+def one_tile(box_scene):
+    """Photons of the paths of one scan tile: step k of a pass of 2048 paths
+    traces paths 2048 k ... of a longer pass's step 0 (the same seeds)."""
+    r = sppm_amd.Renderer(box_scene, scenes.pinhole_camera(8, 8), 0.9, 0.015, SCAN_TILE, bvh_width=8)
+
+    def tile(k):
+        r.begin()  # the slot past a path's last photon is flattened with what an earlier pass left there
+        r.photons(k)
+        r.build()
+        return r.read_path_counts().astype(np.int64), r.read_photons()
+
+    yield tile
     r.close()
+
+
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 4194304, 4194305])
+def test_photon_offsets_scan_sizes(n, box_scene, one_tile):
+    """The stored photons of path counts around a scan tile (2048) and around
+    the tile count where the scan of the tile sums becomes a launch of its own:
+    their number, and in tiles at both ends and between them the photons of
+    every path at the exclusive sum of the counts before it."""
+    r = sppm_amd.Renderer(box_scene, scenes.pinhole_camera(8, 8), 0.9, 0.015, n, bvh_width=8)
+    r.photons(0)
+    stored = r.build()
+    counts = r.read_path_counts().astype(np.int64)
+    assert stored == int(counts.sum())
+    off = np.concatenate([[0], np.cumsum(counts)])
+    ph = r.read_photons()
+    r.close()
+    last = (n - 1) // SCAN_TILE
+    for k in sorted({0, min(1, last), last // 3, last // 2, max(0, last - 1), last}):
+        m = min(SCAN_TILE, n - k * SCAN_TILE)
+        cnt, want = one_tile(k)
+        np.testing.assert_array_equal(counts[k * SCAN_TILE:k * SCAN_TILE + m], cnt[:m])
+        a, q = off[k * SCAN_TILE], int(cnt[:m].sum())
+        for key in ("pos", "flux", "indir"):
+            np.testing.assert_array_equal(ph[key][a:a + q], want[key][:q], err_msg=f"tile {k}: {key}")
