@@ -13,10 +13,10 @@ The defaults (1 warm-up + 255 timed passes) time the configured 256-pass
 render; the radius shrinks from pass to pass, so early passes alone would
 not represent it.
 
-Prints one JSON line.  Extra fields: per-phase kernel times, the roofline of
-the dominant phase (algorithmic bytes per launch / measured launch time,
-hipEvents on the launch stream), and a CPU baseline (the oracle restatement,
-OpenMP, on a bounded sample of the same workload).
+Prints one JSON line.  Extra fields: per-phase kernel times (hipEvents on the
+launch stream), the vector-ALU roofline of the photon pass (counter totals per
+launch / its measured time), the gather's algorithmic rate, and a CPU baseline
+(the oracle restatement, OpenMP, on a bounded sample of the same workload).
 """
 import argparse
 import json
@@ -27,7 +27,6 @@ import time
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, os.path.join(ROOT, "friendsrender-r-public_amd"))
 
-HBM_PEAK_GBS = 8000.0
 # Algorithmic bytes (lower bounds), per unit of work
 STORE_BYTES_PER_PHOTON = 44           # pos 12 + flux 12 + in-dir 12 + pdf 4 + IOR 4
 BUILD_BYTES_PER_PHOTON = 2 * 44 + 8   # one read, one reordered write, key/index
@@ -757,18 +756,17 @@ def main():
     a_hits = (a1["hit_points"] - a0["hit_points"]) / K
     a_nbs = (a1["neighbours"] - a0["neighbours"]) / K
     a_gather = a_hits * GATHER_BYTES_PER_HIT + a_nbs * GATHER_BYTES_PER_NEIGHBOUR
-    # the roofline is given for the gather, the HBM-bound phase with the
-    # largest time; the photon and eye phases are ray traversal (VALU / latency
-    # bound, no HBM roofline) and are reported in phases_ms
     dom = max(("photons", "build", "eye", "gather"), key=lambda k: ms_alone[k])
+    # The gather's algorithmic rate: bytes of every neighbour's record, counted
+    # per pair.  Neighbouring hit points share photons in the caches and LDS, so
+    # it says nothing of the memory's rate (counters of passes 2-4 give its
+    # traffic); the kernel is bound by vector instructions.
     rk = "gather"
-    achieved = algo[rk] / (ms[rk] * 1e-3) / 1e9
-    achieved_alone = a_gather / (ms_alone[rk] * 1e-3) / 1e9
     traffic = read_traffic(os.path.join(ROOT, "profiles", f"traffic_{rk}_{args.workload}.md")) \
         if args.workload == "full" else None
     value = cfg["photons"] * K / el
-    # the photon pass (the longest phase) is neither HBM nor MFMA bound: its
-    # VALU rate, from per-launch counter totals (committed for the BVH8
+    # the roofline is the photon pass' (the longest phase), neither HBM nor MFMA
+    # bound: its VALU rate, from per-launch counter totals (committed for the BVH8
     # megakernel; the photon pass's work does not depend on the radius)
     valu = read_valu(os.path.join(ROOT, "profiles", "valu_pass_kernels_full_material.md")) \
         if args.workload == "full" and cfg["bvh"] == 8 and args.photon_kernel in (None, "megakernel") else {}
@@ -802,18 +800,17 @@ def main():
                    "alpha": cfg["alpha"], "r0": round(cfg["r0"], 6), "camera": cam["type"] and "thin-lens" or "pinhole",
                    "photon_kernel": args.photon_kernel or "default", "wave_bounces": args.wave_bounces or "default",
                    "wave_lanes": args.wave_lanes or "default", "parallelism": "single GPU"},
-        "roofline": {"kernel": rk, "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "algorithmic_bytes_per_launch": int(algo[rk]), "dominant_phase": dom,
-                     "traffic_source": "profiles/traffic_gather_full.md (passes 2-4)" if traffic else None,
-                     "duration": "mean span of the gather phase in the timed passes, beside the next photon pass"},
-        "roofline_alone": {"kernel": rk, "bound": "hbm", "achieved": round(achieved_alone, 1),
-                           "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved_alone / HBM_PEAK_GBS, 4),
-                           "algorithmic_bytes_per_launch": int(a_gather),
-                           "duration": "gather phase alone: the same passes rendered again with the split steps"},
+        "roofline": valu_line,
+        "dominant_phase": dom,
+        "gather_rate": {"bound": "valu", "algorithmic_bytes_per_launch": int(algo[rk]),
+                        "algorithmic_gbs": round(algo[rk] / (ms[rk] * 1e-3) / 1e9, 1),
+                        "algorithmic_gbs_alone": round(a_gather / (ms_alone[rk] * 1e-3) / 1e9, 1),
+                        "hbm_bytes_per_launch_passes_2_4": traffic,
+                        "hbm_source": "profiles/traffic_gather_full.md" if traffic else None,
+                        "duration": "mean span of the gather phase in the timed passes, beside the next photon "
+                                    "pass; alone: the same passes rendered again with the split steps"},
         "phases_ms": {k: round(v, 3) for k, v in ms.items()},
         "phases_alone_ms": {k: round(v, 3) for k, v in ms_alone.items()},
-        "roofline_valu": valu_line,
         "graph_replay": graph_leg,
         "per_pass": {"hit_points": int(hits), "neighbours": int(nbs), "stored_photons": int(stored),
                      "gather_candidates": int(cands), "photon_rays": int(prays), "eye_rays": int(erays),
