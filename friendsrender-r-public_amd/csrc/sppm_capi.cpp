@@ -954,7 +954,7 @@ int sppm_params_set(sppm_ctx* c, const sppm_params* p) {
 // into K segments of L words, K the largest divisor of the block up to 16.
 // Segment k starts k * L words into the stream; after a pass every segment
 // jumps over the K - 1 others.  Every jump costs the same (~10^4 shifted
-// windows), so fewer, longer segments cost less in all; one wave emits a
+// windows), so fewer, longer segments cost less in all; a workgroup emits a
 // segment, and the words are made a pass ahead of their use.
 static int init_camera_stream(sppm_ctx* c) {
     RenderBuffers& R = c->rb;

@@ -2,7 +2,7 @@
 //
 // One pass (SPPM.cpp:770-843):
 //   k_camw_emit/jump shared UniformSample stream words for this pass (K
-//                    segments, each one wave, jump-ahead between passes)
+//                    segments, a workgroup each, jump-ahead between passes)
 //   k_photon<W>      createPhotonMap: persistent, one lane per photon path at
 //                    a time, writes slots
 //   scan(count)      flatten offsets (SPPM.cpp:812-822 order)

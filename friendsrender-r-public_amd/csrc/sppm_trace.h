@@ -19,11 +19,11 @@
 // steps by turns (trav_run); and a leaf's triangles are spread over the lanes
 // (trav_leaves).  With the byte nodes and their one-word sort keys (about 300
 // instructions and 5 loads a node; 900, with a branch per comparator, and 14)
-// the photon pass alone went from 2.80 to 1.97 ms (1M photons, 203k triangles),
+// the photon pass alone went from 2.80 to 1.89 ms (1M photons, 203k triangles),
 // 11.3 to 6.0 ms (4M photons, 500k triangles of rough glass), the eye pass
-// 0.72 to 0.61 and 2.39 to 1.63 ms (1024^2), 1M rays through the 203k triangles
+// 0.72 to 0.58 and 2.39 to 1.64 ms (1024^2), 1M rays through the 203k triangles
 // 0.62 to 0.41 ms, 20k shadow rays 0.078 to 0.053 ms.  (These photon and eye
-// times include the shading's own gains, see lobe_draw.)
+// times include the gains of the shading, see lobe_draw, and of the collapse.)
 //
 // Traversal descends into the nearest intersected child and pushes the
 // others far-to-near.  The first TRACE_LDS stack entries of a lane live in

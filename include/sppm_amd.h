@@ -394,7 +394,8 @@ typedef struct sppm_guide_params {
 #define SPPM_GUIDE_TARGET_MEAN 0
 #define SPPM_GUIDE_TARGET_RMS 1
 /* Parameter count: 64*hidden + hidden + (layers-1)*(hidden*hidden + hidden) + hidden + 1. */
-/* Enable (after sppm_scene_upload) or disable guided emission; re-initialises the weights. */
+/* Enable (after sppm_scene_upload) or disable guided emission; re-initialises the weights.
+ * A failure past the argument checks (no memory) leaves guided emission off. */
 int sppm_guide_set(sppm_ctx* ctx, const sppm_guide_params* params);
 /* Read (out) and/or replace (in, resets Adam) the float32 weights
  * (W1[in][out], b1, ..., W_layers, b_layers, w_out, b_out). */
